@@ -424,12 +424,21 @@ int qmm_gqa_attention(const void* Q, const void* K, const void* V, void* out, in
     if (!Q || !out || (kv_len > 0 && (!K || !V))) return fail(QMM_ERR_INVALID_ARGUMENT, "Q, K, V and Out must be non-null.");
     hipStream_t s = static_cast<hipStream_t>(stream);
     void* part = nullptr;
-    const size_t pb = qmm::attention_workspace_bytes(q_len, num_heads, head_dim, kv_len);
+    // A call of many rows records no pointer into the per-stream scratch when it is captured (a later,
+    // larger call may free it): its keys are not split then.
+    bool may_split = true;
+    if (q_len >= 16) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        may_split = hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+        if (!may_split) (void)hipGetLastError();
+    }
+    const size_t pb = qmm::attention_workspace_bytes(Q, K, V, q_len, kv_len, num_heads, num_kv_heads, head_dim, start_pos,
+                                                     causal != 0, may_split);
     hipError_t e;
     if (pb > 0 && (e = qmm::layer_scratch(s, pb, &part)) != hipSuccess) return hip_fail(e, "attention workspace");
     const float sc = scale != 0.0f ? scale : 1.0f / std::sqrt(static_cast<float>(head_dim));
     e = qmm::launch_attention(Q, K, V, out, part, q_len, kv_len, num_heads, num_kv_heads, head_dim, start_pos, sc,
-                              causal != 0, s);
+                              causal != 0, may_split, s);
     return e == hipSuccess ? QMM_OK : hip_fail(e, "gqa_attention kernel launch");
 }
 
@@ -450,11 +459,9 @@ int qmm_gqa_attention_cached(const void* Q, const void* K_new, const void* V_new
     if (!Q || !K_new || !V_new || !out) return fail(QMM_ERR_INVALID_ARGUMENT, "Q, K_new, V_new and Out must be non-null.");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const size_t row = static_cast<size_t>(num_kv_heads) * head_dim;
-    const size_t bytes = static_cast<size_t>(q_len) * row * 2;
-    hipError_t e;
-    if ((e = hipMemcpyAsync(kc + static_cast<size_t>(start_pos) * row, K_new, bytes, hipMemcpyDeviceToDevice, s)) != hipSuccess ||
-        (e = hipMemcpyAsync(vc + static_cast<size_t>(start_pos) * row, V_new, bytes, hipMemcpyDeviceToDevice, s)) != hipSuccess)
-        return hip_fail(e, "KV cache update");
+    const hipError_t e = qmm::launch_kv_append(K_new, V_new, kc + static_cast<size_t>(start_pos) * row,
+                                               vc + static_cast<size_t>(start_pos) * row, static_cast<int64_t>(q_len) * row, s);
+    if (e != hipSuccess) return hip_fail(e, "KV cache update");
     return qmm_gqa_attention(Q, kc, vc, out, q_len, start_pos + q_len, num_heads, num_kv_heads, head_dim, start_pos, scale,
                              causal, stream);
 }

@@ -148,9 +148,13 @@ hipError_t launch_residual_add(const void* x, const void* r, void* out, int64_t 
 hipError_t launch_swiglu(const void* g, const void* u, void* out, int64_t n, hipStream_t stream);
 hipError_t launch_rope(const void* q, void* q_out, int n_q, const void* k, void* k_out, const void* v, void* v_out, int n_k,
                        int seq_len, int head_dim, int pos_offset, float freq_base, bool neox, hipStream_t stream);
-size_t attention_workspace_bytes(int q_len, int heads, int head_dim, int kv_len);
+// may_split: the matrix-core kernels may cut the keys over workgroups (needs the workspace).
+size_t attention_workspace_bytes(const void* Q, const void* K, const void* V, int q_len, int kv_len, int heads,
+                                 int kv_heads, int head_dim, int start_pos, bool causal, bool may_split);
+// Copies n f16 values of k and of v (one call's new rows) into the cache rows at kc and vc.
+hipError_t launch_kv_append(const void* k, const void* v, void* kc, void* vc, int64_t n, hipStream_t stream);
 hipError_t launch_attention(const void* Q, const void* K, const void* V, void* out, void* part, int q_len, int kv_len,
-                            int heads, int kv_heads, int head_dim, int start_pos, float scale, bool causal,
+                            int heads, int kv_heads, int head_dim, int start_pos, float scale, bool causal, bool may_split,
                             hipStream_t stream);
 LayerStatus kv_cache_init(int layers, int max_seq, int kv_heads, int head_dim);
 LayerStatus kv_cache_free();

@@ -12,12 +12,11 @@
 //   * RoPE: one launch rotates q into its buffer, rotates k straight into the layer's K cache
 //     at the token positions and copies v into the V cache (the reference copies K/V into the
 //     pool separately); inverse frequencies come from the host in fp32, as in the reference.
-//   * Attention: split over the KV length.  A wave owns (query row, query head, chunk of 64
-//     keys): lanes hold head_dim / 64 consecutive query dimensions; keys are loaded 8 at a time
-//     (8 rows in flight per wave), their dot products reduced across the wave together, and an
-//     fp32 online softmax updates the running output.  Chunks are merged in a fixed order by a
-//     second pass (deterministic), skipped for one chunk.  The query heads of one KV head sit
-//     in one workgroup, so their K/V reads share the caches.
+//   * Attention of head_dim 64 and 128 runs on the matrix cores: 16-row tiles for decode and short
+//     calls, 128-row tiles from 16 positions on, the keys split over workgroups where the row tiles
+//     leave the chip idle.  Other head sizes: a wave owns (query row, query head, chunk of 64 keys) on
+//     the vector ALUs.  Ranges are merged in a fixed order by a second pass (deterministic), skipped
+//     for one range.
 //   * SwiGLU and the residual add: 8 values per thread.
 //   * Layer: q/k/v and gate/up each run as one fused projection launch (qmm_gemm_batch), all
 //     kernels on the caller's stream with no host synchronisation; activations live in a
@@ -533,6 +532,22 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const float* __r
     out[idx] = static_cast<_Float16>(sum > 0.0f ? acc / sum : 0.0f);
 }
 
+// Copies the call's new keys and values into their cache rows (one launch for both; two runtime copies
+// took 4.9 us each).  vec: 16-byte pieces, else f16 values.
+__global__ __launch_bounds__(256) void kv_append_kernel(const _Float16* __restrict__ k, const _Float16* __restrict__ v,
+                                                      _Float16* __restrict__ kc, _Float16* __restrict__ vc, int64_t n, int vec) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= n) return;
+    if (vec) {
+        const u32x4 a = reinterpret_cast<const u32x4*>(k)[i], b = reinterpret_cast<const u32x4*>(v)[i];
+        reinterpret_cast<u32x4*>(kc)[i] = a;
+        reinterpret_cast<u32x4*>(vc)[i] = b;
+    } else {
+        kc[i] = k[i];
+        vc[i] = v[i];
+    }
+}
+
 // ---- KV cache pool (one per device) ----------------------------------------------------------
 struct KvPool {
     _Float16* k = nullptr;
@@ -572,6 +587,362 @@ hipError_t layer_workspace(hipStream_t stream, size_t bytes, char** out) {
     return hipSuccess;
 }
 
+// ---- keys split over workgroups ----------------------------------------------------------------
+// Both matrix-core kernels below may cut a row's keys into ranges of `kps` keys, one workgroup each.
+// A range's partial result of row (pos, head) is its running maximum m (base 2), the sum l of its
+// weights 2^(x - m) and the unnormalised output: `o` [split][pos][head][D] and `ml` [split][pos][head]
+// floats.  Ranges past the keys that a row tile sees are neither run nor read.
+struct AttnSplit {
+    float* o;
+    float2* ml;
+    int splits, kps;
+};
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Keys that the rows of a tile of `tile_rows` rows (row r of a KV head's group: position r / group)
+// can see, r any row of the tile.
+__device__ __forceinline__ int tile_keys(int r, int tile_rows, int group, int q_len, int kv_len, int start_pos, int causal) {
+    if (!causal) return kv_len;
+    const int last = min((r / tile_rows * tile_rows + tile_rows - 1) / group, q_len - 1);
+    return min(kv_len, start_pos + last + 1);
+}
+
+// Merges the partial results of each row.  Latency-bound (a few KiB per row): D / 4 threads hold a row's
+// output and `sg` such groups share its ranges, four of them requested at once, so that a decode step's
+// few rows take one or two memory round trips whatever the context; the groups are added in order
+// through LDS.  8B decode at context 4000: 13.0 us with one thread per output element, chunk after chunk.
+template <int D>
+__global__ __launch_bounds__(256) void attention_merge_kernel(AttnSplit sp, _Float16* __restrict__ out, int q_len, int kv_len,
+                                                            int heads, int group, int start_pos, int causal, int tile_rows,
+                                                            int sg) {
+    constexpr int kT = D / 4, kSlots = 256 / kT;
+    __shared__ f32x4 so[kSlots][kT];
+    __shared__ float2 sml[kSlots];
+    const int slot = threadIdx.x / kT, t = threadIdx.x % kT, gi = slot % sg;
+    const int64_t rows = static_cast<int64_t>(q_len) * heads;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * (kSlots / sg) + slot / sg;
+    float m = -INFINITY, l = 0.0f;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (row < rows) {
+        const int pos = static_cast<int>(row / heads), h = static_cast<int>(row % heads);
+        const int n = tile_keys(pos * group + h % group, tile_rows, group, q_len, kv_len, start_pos, causal);
+        const int nv = (n + sp.kps - 1) / sp.kps;
+        for (int c0 = gi; c0 < nv; c0 += 4 * sg) {
+            float2 pm[4];
+            f32x4 po[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int c = c0 + i * sg;
+                const size_t at = static_cast<size_t>(c < nv ? c : c0) * rows + row;
+                pm[i] = sp.ml[at];
+                po[i] = reinterpret_cast<const f32x4*>(sp.o + at * D)[t];
+                if (c >= nv) pm[i] = float2{-INFINITY, 0.0f};
+            }
+            const float mn = fmaxf(fmaxf(fmaxf(pm[0].x, pm[1].x), fmaxf(pm[2].x, pm[3].x)), m);
+            const float a = m == mn ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            l *= a;
+            acc *= a;
+            m = mn;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (c0 + i * sg < nv) {
+                    const float w = __builtin_amdgcn_exp2f(pm[i].x - mn);
+                    l += pm[i].y * w;
+                    acc += po[i] * w;
+                }
+            }
+        }
+    }
+    if (sg > 1) {
+        so[slot][t] = acc;
+        if (t == 0) sml[slot] = float2{m, l};
+        __syncthreads();
+        if (gi != 0) return;
+        for (int i = 1; i < sg; ++i) {
+            const float2 o = sml[slot + i];
+            if (o.x == -INFINITY && o.y == 0.0f) continue;  // a group without ranges
+            const float mn = fmaxf(m, o.x);
+            const float a = m == mn ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            const float b = __builtin_amdgcn_exp2f(o.x - mn);
+            l = l * a + o.y * b;
+            acc = acc * a + so[slot + i][t] * b;
+            m = mn;
+        }
+    }
+    if (row >= rows) return;
+    _Float16 h4[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) h4[i] = static_cast<_Float16>(acc[i] / l);
+    __builtin_memcpy(out + row * D + 4 * t, h4, 8);
+}
+
+// ---- few query rows on the matrix cores ---------------------------------------------------------
+// Attention of up to 16 rows (positions x query heads of one KV head) against one KV head's keys: the
+// decode step, short chunks, and query groups that do not divide the 128-row tile below.  Bound by
+// reading K and V (each once per row tile, whatever the number of query heads) and by the latency of
+// one pass.  A wave takes 32 keys at a time, no LDS on the way:
+//   * S^T = K Q^T on v_mfma_f32_16x16x32_f16: lane (l, q) = (lane % 16, lane / 16) loads 16 bytes of
+//     key l's row per 32 dims (4 lanes read 64 contiguous bytes) and receives the scores of row l
+//     with keys 4q..4q+3 of each 16-key tile;
+//   * those 8 keys are the k order of the second product's operand, so the weights go straight from
+//     the score registers into O^T += V^T P^T; lane (l, q) loads dims D/16 l .. of its 8 keys' V rows
+//     (16 lanes read one whole row) and v_perm transposes them in registers;
+//   * weights stay at fp32 precision: 2^10 p = hi + lo in f16, two products (the scale keeps lo clear
+//     of f16's subnormals; it cancels against the sum).
+// The 4 waves of a workgroup take every fourth 32-key block of its range and are merged through LDS in
+// wave order.  8B decode at context 4000 (16 MB of keys and values): 7.8 us and 4.3 us of merge, against
+// 12.2 us and 13.0 us with one wave per (query head, 64 keys) on the vector ALUs, which reads each
+// row once per query head and leaves four times the partial results.
+// With kRope (one query position, the decode step): Q, k_new and v_new are the projections before RoPE.
+// The rotation runs on the operand registers; the new key (position start_pos) and its value are taken
+// from k_new / v_new, and the workgroup of row tile 0 whose range ends with it writes both into the
+// cache row, which no lane of the launch reads.
+constexpr int kRowsTile = 16, kRowsKeys = 32, kRowsWaves = 4;
+
+template <int D>
+__device__ __forceinline__ void rotate_row(f16x8 (&f)[D / 32], const DecodeRope& dr, int q) {
+    if (dr.neox) {
+#pragma unroll
+        for (int db = 0; db < D / 64; ++db)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int p = 32 * db + 8 * q + e;
+                const float cs = dr.cs[p], sn = dr.sn[p];
+                const float a = static_cast<float>(f[db][e]), b = static_cast<float>(f[db + D / 64][e]);
+                f[db][e] = static_cast<_Float16>(a * cs - b * sn);
+                f[db + D / 64][e] = static_cast<_Float16>(a * sn + b * cs);
+            }
+    } else {
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int p = 16 * db + 4 * q + e;
+                const float cs = dr.cs[p], sn = dr.sn[p];
+                const float a = static_cast<float>(f[db][2 * e]), b = static_cast<float>(f[db][2 * e + 1]);
+                f[db][2 * e] = static_cast<_Float16>(a * cs - b * sn);
+                f[db][2 * e + 1] = static_cast<_Float16>(a * sn + b * cs);
+            }
+    }
+}
+
+template <int D, bool kRope>
+__global__ __launch_bounds__(64 * kRowsWaves) void attention_rows_kernel(
+    const _Float16* __restrict__ Q, const _Float16* __restrict__ Kc, const _Float16* __restrict__ Vc, _Float16* __restrict__ out,
+    AttnSplit sp, int q_len, int kv_len, int heads, int kv_heads, int start_pos, float scale_log2, int causal, int rtiles,
+    DecodeRope dr) {
+    constexpr int kVW = D / 32;  // dwords of a lane's V slice: dims D/16 l .. D/16 l + D/16 - 1
+    constexpr float kPScale = 10.0f;
+    const int group = heads / kv_heads;
+    const int g = static_cast<int>(blockIdx.x % kv_heads);
+    const int rest = static_cast<int>(blockIdx.x / kv_heads);
+    const int rt = rest % rtiles, split = rest / rtiles;
+    const int n_rows = q_len * group;
+    const int n_keys = tile_keys(rt * kRowsTile, kRowsTile, group, q_len, kv_len, start_pos, causal);
+    const int k_begin = split * sp.kps, k_end = min(n_keys, k_begin + sp.kps);
+    if (k_begin >= n_keys) return;
+    const int lane = threadIdx.x & 63, l = lane & 15, q = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = min(rt * kRowsTile + l, n_rows - 1);  // rows past the last repeat it
+    const int pos = r / group, head = g * group + r % group;
+    const int row_end = causal ? min(kv_len, start_pos + pos + 1) : kv_len;  // keys this row sees
+    const int vis_all = causal ? min(kv_len, start_pos + rt * kRowsTile / group + 1) : kv_len;  // keys every row sees
+    const size_t kv_row = static_cast<size_t>(kv_heads) * D;
+    const _Float16* kbase = Kc + static_cast<size_t>(g) * D;
+    const _Float16* vbase = Vc + static_cast<size_t>(g) * D;
+
+    f16x8 qf[D / 32];
+    {
+        const _Float16* qrow = Q + (static_cast<size_t>(pos) * heads + head) * D + 8 * q;
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db) qf[db] = *reinterpret_cast<const f16x8*>(qrow + 32 * db);
+        if constexpr (kRope) rotate_row<D>(qf, dr, q);
+    }
+    f32x4 o[D / 16];
+#pragma unroll
+    for (int dt = 0; dt < D / 16; ++dt) o[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    float m_run = -INFINITY, l_run = 0.0f;
+
+    for (int kb = k_begin + kRowsKeys * w; kb < k_end; kb += kRowsKeys * kRowsWaves) {
+        // keys past the tile's last read that key; their weights are zero
+        f16x8 kf[2][D / 32];
+        uint32_t vd[8][kVW];  // V slices of keys kb + 16 (j / 4) + 4 q + j % 4
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            const int k = min(kb + 16 * tt + l, n_keys - 1);
+            const _Float16* kr = kbase + static_cast<size_t>(k) * kv_row + 8 * q;
+            if constexpr (kRope)
+                if (k == start_pos) kr = dr.k_new + static_cast<size_t>(g) * D + 8 * q;
+#pragma unroll
+            for (int db = 0; db < D / 32; ++db) kf[tt][db] = *reinterpret_cast<const f16x8*>(kr + 32 * db);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int k = min(kb + 16 * (j >> 2) + 4 * q + (j & 3), n_keys - 1);
+            const _Float16* vr = vbase + static_cast<size_t>(k) * kv_row;
+            if constexpr (kRope)
+                if (k == start_pos) vr = dr.v_new + static_cast<size_t>(g) * D;
+            __builtin_memcpy(vd[j], __builtin_assume_aligned(vr + D / 16 * l, D / 8), 4 * kVW);
+        }
+        if constexpr (kRope) {
+            if (kb + kRowsKeys > start_pos) {  // the block with the new key
+#pragma unroll
+                for (int tt = 0; tt < 2; ++tt) {
+                    const bool is_new = min(kb + 16 * tt + l, n_keys - 1) == start_pos;
+                    f16x8 rot[D / 32];
+#pragma unroll
+                    for (int db = 0; db < D / 32; ++db) rot[db] = kf[tt][db];
+                    rotate_row<D>(rot, dr, q);
+#pragma unroll
+                    for (int db = 0; db < D / 32; ++db) kf[tt][db] = is_new ? rot[db] : kf[tt][db];
+                    if (rt == 0 && kb + 16 * tt + l == start_pos) {
+                        _Float16* kw = dr.kc + static_cast<size_t>(start_pos) * kv_row + static_cast<size_t>(g) * D + 8 * q;
+#pragma unroll
+                        for (int db = 0; db < D / 32; ++db) *reinterpret_cast<f16x8*>(kw + 32 * db) = rot[db];
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (rt == 0 && kb + 16 * (j >> 2) + 4 * q + (j & 3) == start_pos) {
+                        _Float16* vw = dr.vc + static_cast<size_t>(start_pos) * kv_row + static_cast<size_t>(g) * D + D / 16 * l;
+                        __builtin_memcpy(__builtin_assume_aligned(vw, D / 8), vd[j], 4 * kVW);
+                    }
+            }
+        }
+        // scores: x[4 tt + v] of key kb + 16 tt + 4 q + v
+        const bool full = kb + kRowsKeys <= vis_all;
+        float x[8];
+        float mx = -INFINITY;
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int db = 0; db < D / 32; ++db) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[tt][db], qf[db], s, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                float y = s[v] * scale_log2;
+                if (!full && kb + 16 * tt + 4 * q + v >= row_end) y = -INFINITY;
+                x[4 * tt + v] = y;
+                mx = fmaxf(mx, y);
+            }
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        // a row that sees no key of this block keeps its state (its maximum may still be -inf)
+        const bool sees = kb < row_end;
+        const float m_new = sees ? fmaxf(m_run, mx) : m_run;
+        const float corr = sees ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
+        const float base = sees ? m_new - kPScale : 0.0f;
+        float sum = 0.0f;
+        f16x8 ph, pl;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float p = __builtin_amdgcn_exp2f(x[i] - base);
+            sum += p;
+            ph[i] = static_cast<_Float16>(p);
+            pl[i] = static_cast<_Float16>(p - static_cast<float>(ph[i]));
+        }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        l_run = l_run * corr + sum;
+        m_run = m_new;
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) o[dt] *= corr;
+        // product dt: operand row l is dim D/16 l + dt of the lane's 8 keys
+        auto pv = [&](const uint32_t (&v)[8][kVW], f32x4 (&acc)[D / 16]) {
+#pragma unroll
+            for (int dt = 0; dt < D / 16; ++dt) {
+                uint32_t t[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    t[i] = __builtin_amdgcn_perm(v[2 * i + 1][dt >> 1], v[2 * i][dt >> 1], (dt & 1) ? 0x07060302u : 0x05040100u);
+                f16x8 vf;
+                __builtin_memcpy(&vf, t, 16);
+                acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph, acc[dt], 0, 0, 0);
+                acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl, acc[dt], 0, 0, 0);
+            }
+        };
+        bool plain = true;
+        if (!full) {
+            // some row does not see some key: its weight 0 must not meet an infinite or NaN value
+            bool bad = false;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int i = 0; i < kVW; ++i)
+                    bad |= (vd[j][i] & 0x7C00u) == 0x7C00u || (vd[j][i] & 0x7C000000u) == 0x7C000000u;
+            plain = __ballot(bad) == 0;
+        }
+        if (plain) {
+            pv(vd, o);
+        } else {
+            // one row at a time, with the values that it does not see cleared
+            for (int rr = 0; rr < kRowsTile; ++rr) {
+                const int end = __shfl(row_end, rr, 64);
+                uint32_t vz[8][kVW];
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+#pragma unroll
+                    for (int i = 0; i < kVW; ++i) vz[j][i] = kb + 16 * (j >> 2) + 4 * q + (j & 3) < end ? vd[j][i] : 0u;
+                f32x4 t[D / 16];
+#pragma unroll
+                for (int dt = 0; dt < D / 16; ++dt) t[dt] = o[dt];
+                pv(vz, t);
+#pragma unroll
+                for (int dt = 0; dt < D / 16; ++dt) o[dt] = l == rr ? t[dt] : o[dt];
+            }
+        }
+    }
+
+    // Lane (l, q) holds dims D/4 q + D/16 v + dt of row l in o[dt][v].  Merge of the waves: LDS rows
+    // padded by one 16-byte piece.
+    constexpr int kRowF = D + 4;
+    __shared__ __align__(16) float so[kRowsWaves][kRowsTile * kRowF];
+    __shared__ float2 sml[kRowsWaves][kRowsTile];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int dt = 0; dt < D / 16; dt += 4)
+            *reinterpret_cast<f32x4*>(&so[w][l * kRowF + D / 4 * q + D / 16 * v + dt]) =
+                f32x4{o[dt][v], o[dt + 1][v], o[dt + 2][v], o[dt + 3][v]};
+    if (q == 0) sml[w][l] = float2{m_run, l_run};
+    __syncthreads();
+    constexpr int kPer = D / 16;  // dims per thread: 16 threads per row
+    const int mr = threadIdx.x >> 4, d0 = kPer * (threadIdx.x & 15);
+    const int row = rt * kRowsTile + mr;
+    if (row >= n_rows) return;
+    float mm = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < kRowsWaves; ++i) mm = fmaxf(mm, sml[i][mr].x);
+    float ls = 0.0f;
+    f32x4 acc[kPer / 4];
+#pragma unroll
+    for (int j = 0; j < kPer / 4; ++j) acc[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < kRowsWaves; ++i) {
+        const float2 ml = sml[i][mr];
+        if (ml.x == -INFINITY && ml.y == 0.0f) continue;  // no key seen
+        const float a = __builtin_amdgcn_exp2f(ml.x - mm);
+        ls += ml.y * a;
+#pragma unroll
+        for (int j = 0; j < kPer / 4; ++j) acc[j] += *reinterpret_cast<const f32x4*>(&so[i][mr * kRowF + d0 + 4 * j]) * a;
+    }
+    const size_t orow = static_cast<size_t>(row / group) * heads + g * group + row % group;
+    if (sp.splits == 1) {
+        _Float16 hv[kPer];
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) hv[j] = static_cast<_Float16>(acc[j / 4][j % 4] / ls);
+        __builtin_memcpy(out + orow * D + d0, hv, 2 * kPer);
+    } else {
+        const size_t at = static_cast<size_t>(split) * q_len * heads + orow;
+#pragma unroll
+        for (int j = 0; j < kPer / 4; ++j) *reinterpret_cast<f32x4*>(sp.o + at * D + d0 + 4 * j) = acc[j];
+        if (d0 == 0) sp.ml[at] = float2{mm, ls};
+    }
+}
+
 // ---- prefill attention on the matrix cores --------------------------------------------------
 // Flash-attention form for many query rows.  A workgroup of 4 waves owns 128 query rows: the
 // 128 / G positions of a position tile times the G query heads of one KV head, which share every
@@ -589,8 +960,6 @@ hipError_t layer_workspace(hipStream_t stream, size_t bytes, char** out) {
 // first (causal rows near the end see the most keys); with 8 KV heads the workgroups of one KV
 // head land on one XCD and share its L2.
 constexpr int kFaRows = 128, kFaKeys = 64, kFaThreads = 256;
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 template <int D>
 struct FaGeom {
@@ -611,13 +980,14 @@ extern __shared__ __align__(16) _Float16 fa_lds[];
 template <int D>
 __global__ __launch_bounds__(kFaThreads, 2) void attention_mfma_kernel(
     const _Float16* __restrict__ Q, const _Float16* __restrict__ Kc, const _Float16* __restrict__ Vc,
-    _Float16* __restrict__ out, int q_len, int kv_len, int heads, int kv_heads, int start_pos, float scale_log2,
-    int causal, int ptiles) {
+    _Float16* __restrict__ out, AttnSplit sp, int q_len, int kv_len, int heads, int kv_heads, int start_pos,
+    float scale_log2, int causal, int ptiles) {
     using FG = FaGeom<D>;
     const int group = heads / kv_heads;
     const int ppw = kFaRows / group;  // positions per workgroup
     const int g = static_cast<int>(blockIdx.x % kv_heads);
-    const int pt = ptiles - 1 - static_cast<int>(blockIdx.x / kv_heads);
+    const int pt = ptiles - 1 - static_cast<int>(blockIdx.x / kv_heads) % ptiles;
+    const int split = static_cast<int>(blockIdx.x / kv_heads) / ptiles;
     const int p0 = pt * ppw;
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
     const int r = 32 * (tid >> 6) + l32;  // row of the workgroup
@@ -625,7 +995,9 @@ __global__ __launch_bounds__(kFaThreads, 2) void attention_mfma_kernel(
     const int head = g * group + r % group;
     const int p_last = min(p0 + ppw, q_len) - 1;
     const int n_keys = causal ? min(kv_len, start_pos + p_last + 1) : kv_len;
-    const int n_tiles = (n_keys + kFaKeys - 1) / kFaKeys;
+    const int t0 = split * (sp.kps / kFaKeys);
+    const int n_tiles = min((n_keys + kFaKeys - 1) / kFaKeys, t0 + sp.kps / kFaKeys);
+    if (t0 >= n_tiles) return;
     const int vis_all = causal ? min(kv_len, start_pos + p0 + 1) : kv_len;    // keys every row sees
     const int row_end = causal ? min(kv_len, start_pos + pos + 1) : kv_len;   // keys this row sees
     const size_t kv_row = static_cast<size_t>(kv_heads) * D;
@@ -689,11 +1061,18 @@ __global__ __launch_bounds__(kFaThreads, 2) void attention_mfma_kernel(
         for (int v = 0; v < 16; ++v) o[dt][v] = 0.0f;
     float m_run = -INFINITY, l_run = 0.0f;
 
-    load(0);
-    store(0);
+    // waves whose 32 rows all lie past q_len only stage
+    const bool live = p0 + __builtin_amdgcn_readfirstlane(32 * (tid >> 6)) / group < q_len;
+    load(t0);
+    store(t0 & 1);
     __syncthreads();
-    for (int t = 0; t < n_tiles; ++t) {
+    for (int t = t0; t < n_tiles; ++t) {
         if (t + 1 < n_tiles) load(t + 1);
+        if (!live) {
+            if (t + 1 < n_tiles) store((t + 1) & 1);
+            __syncthreads();
+            continue;
+        }
         const _Float16* sk = fa_lds + (t & 1) * FG::kBuf;
         const _Float16* sv = sk + FG::kK;
         // S^T tiles: register v of tile tt is key 32 tt + 8 (v / 4) + 4 h + v % 4 of the row l32
@@ -722,24 +1101,29 @@ __global__ __launch_bounds__(kFaThreads, 2) void attention_mfma_kernel(
                 mx = fmaxf(mx, x);
             }
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fmaxf(m_run, mx);  // finite: key 0 is visible to every row
-        const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
+        // a row that sees no key of this tile keeps its state (its maximum may still be -inf)
+        const bool sees = kb < row_end;
+        const float m_new = sees ? fmaxf(m_run, mx) : m_run;
+        const float corr = sees ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
+        const float base = sees ? m_new : 0.0f;
         float sum = 0.0f;
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                const float p = __builtin_amdgcn_exp2f(s[tt][v] - m_new);
+                const float p = __builtin_amdgcn_exp2f(s[tt][v] - base);
                 s[tt][v] = p;
                 sum += p;
             }
         sum += __shfl_xor(sum, 32, 64);
         l_run = l_run * corr + sum;
         m_run = m_new;
+        if (__ballot(corr != 1.0f) != 0) {  // some row's maximum grew
 #pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
+            for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) o[dt][v] *= corr;
+                for (int v = 0; v < 16; ++v) o[dt][v] *= corr;
+        }
         // 16-key block b: lane half h holds keys 16 b + 4 h + (0..3) and 16 b + 8 + 4 h + (0..3)
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
@@ -759,7 +1143,17 @@ __global__ __launch_bounds__(kFaThreads, 2) void attention_mfma_kernel(
         __syncthreads();
     }
 
-    if (pos < q_len) {
+    if (pos >= q_len) return;
+    if (sp.splits > 1) {
+        const size_t at = (static_cast<size_t>(split) * q_len + pos) * heads + head;
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4)
+                *reinterpret_cast<f32x4*>(sp.o + at * D + 32 * dt + 8 * q4 + 4 * h) =
+                    f32x4{o[dt][4 * q4], o[dt][4 * q4 + 1], o[dt][4 * q4 + 2], o[dt][4 * q4 + 3]};
+        if (h == 0) sp.ml[at] = float2{m_run, l_run};
+    } else {
         const float inv = 1.0f / l_run;
         _Float16* orow = out + (static_cast<size_t>(pos) * heads + head) * D;
 #pragma unroll
@@ -776,9 +1170,80 @@ __global__ __launch_bounds__(kFaThreads, 2) void attention_mfma_kernel(
 
 int attn_chunks(int kv_len) { return kv_len <= 0 ? 1 : (kv_len + kAttnChunk - 1) / kAttnChunk; }
 
-size_t attn_part_bytes(int q_len, int heads, int head_dim, int kv_len) {
-    const int ch = attn_chunks(kv_len);
-    return ch > 1 ? static_cast<size_t>(q_len) * heads * ch * (head_dim + 2) * sizeof(float) : 0;
+// Which attention kernel serves a call, and how its keys are split over workgroups.
+//   kMfma: >= kFaMinRows query positions (fewer leave the 128-row tile mostly empty) of a query group
+//          that divides 128;
+//   kRows: the other calls of head_dim 64 and 128;
+//   kLanes: other head sizes, and Q / K / V that are not 16-byte aligned.
+constexpr int kFaMinRows = 16;
+// Workgroups that a split grid is cut to: two per CU, what the 128-row tile's LDS allows.
+constexpr int64_t kAttnFill = 512;
+enum class AttnKind { kMfma, kRows, kLanes };
+struct AttnPlan {
+    AttnKind kind;
+    int tile_rows, tiles;  // rows per tile (positions x query heads of a KV head), row tiles
+    int splits, kps;       // key ranges per row tile and keys per range
+    size_t bytes;          // workspace of the partial results
+};
+
+// Keys per range: the key blocks of all row tiles spread over kAttnFill workgroups (a block: 64 keys of
+// the 128-row tile, at least two per range, or 32 keys of each wave of the 16-row tile).  A tile's keys
+// are split only while the grid leaves half of the workgroups' places empty: partial results cost
+// 4 D bytes of traffic per row, range and direction.  40 positions of 32 heads over 12040 keys (16
+// row tiles of 128): 30 us and 6.7 us of merge in 32 ranges, against 405 us unsplit.
+AttnPlan attn_plan(int q_len, int kv_len, int heads, int kv_heads, int head_dim, int start_pos, bool causal, bool aligned,
+                   bool may_split) {
+    const int group = heads / kv_heads;
+    const int64_t rows = static_cast<int64_t>(q_len) * group;
+    const size_t row_bytes = static_cast<size_t>(q_len) * heads * (head_dim + 2) * sizeof(float);
+    AttnPlan p{};
+    if ((head_dim != 64 && head_dim != 128) || kv_len <= 0 || !aligned || rows > (1 << 30)) {
+        p.kind = AttnKind::kLanes;
+        p.splits = attn_chunks(kv_len);
+        p.kps = kAttnChunk;
+        p.bytes = p.splits > 1 ? row_bytes * p.splits : 0;
+        return p;
+    }
+    const bool mfma = q_len >= kFaMinRows && kFaRows % group == 0;
+    p.kind = mfma ? AttnKind::kMfma : AttnKind::kRows;
+    p.tile_rows = mfma ? kFaRows : kRowsTile;
+    p.tiles = static_cast<int>((rows + p.tile_rows - 1) / p.tile_rows);
+    const int block = mfma ? kFaKeys : kRowsKeys * kRowsWaves;
+    const int64_t wgs = static_cast<int64_t>(p.tiles) * kv_heads;
+    int64_t blocks = 0;  // of one KV head
+    int most = 0;        // of one row tile
+    for (int t = 0; t < p.tiles; ++t) {
+        int n = kv_len;
+        if (causal) {
+            const int64_t last = std::min((static_cast<int64_t>(t + 1) * p.tile_rows - 1) / group, static_cast<int64_t>(q_len) - 1);
+            n = static_cast<int>(std::min<int64_t>(kv_len, start_pos + last + 1));
+        }
+        const int b = (n + block - 1) / block;
+        blocks += b;
+        most = std::max(most, b);
+    }
+    int per = most;
+    if (may_split && 2 * wgs <= kAttnFill) {
+        const int64_t even = (blocks * kv_heads + kAttnFill - 1) / kAttnFill;
+        per = static_cast<int>(std::min<int64_t>(most, std::max<int64_t>(even, mfma ? 2 : 1)));
+    }
+    p.splits = (most + per - 1) / per;
+    p.kps = per * block;
+    p.bytes = p.splits > 1 ? row_bytes * p.splits : 0;
+    return p;
+}
+
+AttnSplit attn_split(const AttnPlan& p, void* part, int q_len, int heads, int head_dim) {
+    AttnSplit sp{};
+    sp.splits = p.splits;
+    sp.kps = p.kps;
+    sp.o = static_cast<float*>(part);
+    if (p.splits > 1) sp.ml = reinterpret_cast<float2*>(sp.o + static_cast<size_t>(p.splits) * q_len * heads * head_dim);
+    return sp;
+}
+
+bool attn_aligned(const void* Q, const void* K, const void* V) {
+    return (reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V)) % 16 == 0;
 }
 
 }  // namespace
@@ -831,20 +1296,35 @@ hipError_t launch_rope(const void* q, void* q_out, int n_q, const void* k, void*
     return hipGetLastError();
 }
 
-size_t attention_workspace_bytes(int q_len, int heads, int head_dim, int kv_len) {
-    return attn_part_bytes(q_len, heads, head_dim, kv_len);
+size_t attention_workspace_bytes(const void* Q, const void* K, const void* V, int q_len, int kv_len, int heads,
+                                 int kv_heads, int head_dim, int start_pos, bool causal, bool may_split) {
+    const bool al = attn_aligned(Q, K, V);
+    const AttnPlan p = attn_plan(q_len, kv_len, heads, kv_heads, head_dim, std::min(start_pos, kv_len), causal, al, may_split);
+    return p.bytes;
 }
 
 namespace {
 
-// The matrix-core kernel serves head_dim 64 and 128, query groups dividing 128, at least
-// kFaMinRows query positions (fewer rows leave the 32-row MFMA tiles mostly empty) and 16-byte
-// aligned Q / K / V.
-constexpr int kFaMinRows = 16;
+hipError_t launch_merge(const AttnPlan& p, const AttnSplit& sp, _Float16* out, int q_len, int kv_len, int heads, int kv_heads,
+                        int head_dim, int start_pos, bool causal, hipStream_t stream) {
+    const int64_t rows = static_cast<int64_t>(q_len) * heads;
+    const int slots = 1024 / head_dim;
+    int sg = 1;  // groups of threads per row: four ranges each, as long as the rows leave CUs idle
+    while (sg < slots && 4 * sg < p.splits && rows * sg < 8192) sg *= 2;
+    const int64_t blocks = (rows * sg + slots - 1) / slots;
+    auto go = [&](auto dc) {
+        hipLaunchKernelGGL((attention_merge_kernel<decltype(dc)::value>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, sp,
+                           out, q_len, kv_len, heads, heads / kv_heads, start_pos, causal ? 1 : 0, p.tile_rows, sg);
+    };
+    if (head_dim == 128) go(std::integral_constant<int, 128>{});
+    else go(std::integral_constant<int, 64>{});
+    return hipGetLastError();
+}
 
 template <int D>
-hipError_t launch_attention_mfma(const void* Q, const void* K, const void* V, void* out, int q_len, int kv_len, int heads,
-                                 int kv_heads, int start_pos, float scale, bool causal, hipStream_t stream) {
+hipError_t launch_attention_mfma(const AttnPlan& p, const AttnSplit& sp, const void* Q, const void* K, const void* V, void* out,
+                                 int q_len, int kv_len, int heads, int kv_heads, int start_pos, float scale, bool causal,
+                                 hipStream_t stream) {
     using FG = FaGeom<D>;
     static std::once_flag once;
     static hipError_t attr = hipSuccess;
@@ -853,33 +1333,61 @@ hipError_t launch_attention_mfma(const void* Q, const void* K, const void* V, vo
                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(FG::kLdsBytes));
     });
     if (attr != hipSuccess) return attr;
-    const int ppw = kFaRows / (heads / kv_heads);
-    const int ptiles = (q_len + ppw - 1) / ppw;
     const float scale_log2 = scale * 1.4426950408889634f;
-    hipLaunchKernelGGL((attention_mfma_kernel<D>), dim3(static_cast<unsigned>(ptiles * kv_heads)), dim3(kFaThreads),
+    hipLaunchKernelGGL((attention_mfma_kernel<D>), dim3(static_cast<unsigned>(p.tiles * kv_heads * p.splits)), dim3(kFaThreads),
                        FG::kLdsBytes, stream, static_cast<const _Float16*>(Q), static_cast<const _Float16*>(K),
-                       static_cast<const _Float16*>(V), static_cast<_Float16*>(out), q_len, kv_len, heads, kv_heads,
-                       start_pos, scale_log2, causal ? 1 : 0, ptiles);
+                       static_cast<const _Float16*>(V), static_cast<_Float16*>(out), sp, q_len, kv_len, heads, kv_heads,
+                       start_pos, scale_log2, causal ? 1 : 0, p.tiles);
     return hipGetLastError();
 }
 
-bool attention_mfma_ok(const void* Q, const void* K, const void* V, int q_len, int kv_len, int heads, int kv_heads,
-                       int head_dim) {
-    const bool aligned = (reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V)) % 16 == 0;
-    const int group = heads / kv_heads;
-    return (head_dim == 64 || head_dim == 128) && kFaRows % group == 0 && q_len >= kFaMinRows && kv_len > 0 && aligned;
+template <int D, bool kRope>
+hipError_t launch_attention_rows(const AttnPlan& p, const AttnSplit& sp, const void* Q, const void* K, const void* V, void* out,
+                                 int q_len, int kv_len, int heads, int kv_heads, int start_pos, float scale, bool causal,
+                                 const DecodeRope& dr, hipStream_t stream) {
+    const int64_t blocks = static_cast<int64_t>(p.tiles) * kv_heads * p.splits;
+    if (blocks > INT32_MAX) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL((attention_rows_kernel<D, kRope>), dim3(static_cast<unsigned>(blocks)), dim3(64 * kRowsWaves), 0, stream,
+                       static_cast<const _Float16*>(Q), static_cast<const _Float16*>(K), static_cast<const _Float16*>(V),
+                       static_cast<_Float16*>(out), sp, q_len, kv_len, heads, kv_heads, start_pos,
+                       scale * 1.4426950408889634f, causal ? 1 : 0, p.tiles, dr);
+    return hipGetLastError();
 }
 
 }  // namespace
 
+hipError_t launch_kv_append(const void* k, const void* v, void* kc, void* vc, int64_t n, hipStream_t stream) {
+    if (n <= 0) return hipSuccess;
+    const uintptr_t al = reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(kc) |
+                         reinterpret_cast<uintptr_t>(vc);
+    const bool vec = al % 16 == 0 && n % 8 == 0;
+    const int64_t items = vec ? n / 8 : n;
+    hipLaunchKernelGGL(kv_append_kernel, dim3(static_cast<unsigned>((items + 255) / 256)), dim3(256), 0, stream,
+                       static_cast<const _Float16*>(k), static_cast<const _Float16*>(v), static_cast<_Float16*>(kc),
+                       static_cast<_Float16*>(vc), items, vec ? 1 : 0);
+    return hipGetLastError();
+}
+
 hipError_t launch_attention(const void* Q, const void* K, const void* V, void* out, void* part, int q_len, int kv_len,
-                            int heads, int kv_heads, int head_dim, int start_pos, float scale, bool causal,
+                            int heads, int kv_heads, int head_dim, int start_pos, float scale, bool causal, bool may_split,
                             hipStream_t stream) {
     if (q_len <= 0 || heads <= 0) return hipSuccess;
-    if (attention_mfma_ok(Q, K, V, q_len, kv_len, heads, kv_heads, head_dim)) {
-        if (head_dim == 128)
-            return launch_attention_mfma<128>(Q, K, V, out, q_len, kv_len, heads, kv_heads, start_pos, scale, causal, stream);
-        return launch_attention_mfma<64>(Q, K, V, out, q_len, kv_len, heads, kv_heads, start_pos, scale, causal, stream);
+    const bool aligned = attn_aligned(Q, K, V);
+    start_pos = std::min(start_pos, kv_len);  // every row sees all keys from there on
+    const AttnPlan p = attn_plan(q_len, kv_len, heads, kv_heads, head_dim, start_pos, causal, aligned, may_split);
+    hipError_t e;
+    if (p.kind != AttnKind::kLanes) {
+        const AttnSplit sp = attn_split(p, part, q_len, heads, head_dim);
+        auto go = [&](auto dc) {
+            constexpr int D = decltype(dc)::value;
+            return p.kind == AttnKind::kMfma
+                       ? launch_attention_mfma<D>(p, sp, Q, K, V, out, q_len, kv_len, heads, kv_heads, start_pos, scale, causal, stream)
+                       : launch_attention_rows<D, false>(p, sp, Q, K, V, out, q_len, kv_len, heads, kv_heads, start_pos, scale,
+                                                         causal, DecodeRope{}, stream);
+        };
+        e = head_dim == 128 ? go(std::integral_constant<int, 128>{}) : go(std::integral_constant<int, 64>{});
+        if (e != hipSuccess || p.splits == 1) return e;
+        return launch_merge(p, sp, static_cast<_Float16*>(out), q_len, kv_len, heads, kv_heads, head_dim, start_pos, causal, stream);
     }
     const int chunks = attn_chunks(kv_len);
     const int64_t waves = static_cast<int64_t>(q_len) * heads * chunks;
@@ -891,7 +1399,6 @@ hipError_t launch_attention(const void* Q, const void* K, const void* V, void* o
                            static_cast<float*>(part), q_len, kv_len, heads, kv_heads, head_dim, start_pos, scale,
                            causal ? 1 : 0, chunks);
     };
-    const bool aligned = (reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V)) % 16 == 0;
     if (head_dim % 8 == 0 && head_dim <= 128 && aligned)
         hipLaunchKernelGGL((attention_keys_kernel<false>), grid, dim3(256), 0, stream, static_cast<const _Float16*>(Q),
                            static_cast<const _Float16*>(K), static_cast<const _Float16*>(V), static_cast<_Float16*>(out),
@@ -900,7 +1407,7 @@ hipError_t launch_attention(const void* Q, const void* K, const void* V, void* o
     else if (head_dim <= 64) go(std::integral_constant<int, 1>{});
     else if (head_dim <= 128) go(std::integral_constant<int, 2>{});
     else go(std::integral_constant<int, 4>{});
-    hipError_t e = hipGetLastError();
+    e = hipGetLastError();
     if (e != hipSuccess || chunks == 1) return e;
     const int64_t n = static_cast<int64_t>(q_len) * heads * head_dim;
     hipLaunchKernelGGL(attention_combine_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, stream,
@@ -928,7 +1435,17 @@ hipError_t launch_attention_decode_rope(const void* q, const void* k_new, const 
         dr.cs[i] = static_cast<float>(std::cos(static_cast<double>(ang)));
         dr.sn[i] = static_cast<float>(std::sin(static_cast<double>(ang)));
     }
-    const int chunks = attn_chunks(kv_len);
+    const AttnPlan p = attn_plan(1, kv_len, heads, kv_heads, head_dim, kv_len - 1, true, true, true);
+    if (p.kind == AttnKind::kRows) {
+        const AttnSplit sp = attn_split(p, part, 1, heads, head_dim);
+        const hipError_t e = head_dim == 128 ? launch_attention_rows<128, true>(p, sp, q, kc, vc, out, 1, kv_len, heads, kv_heads,
+                                                                                kv_len - 1, scale, true, dr, stream)
+                                             : launch_attention_rows<64, true>(p, sp, q, kc, vc, out, 1, kv_len, heads, kv_heads,
+                                                                               kv_len - 1, scale, true, dr, stream);
+        if (e != hipSuccess || p.splits == 1) return e;
+        return launch_merge(p, sp, static_cast<_Float16*>(out), 1, kv_len, heads, kv_heads, head_dim, kv_len - 1, true, stream);
+    }
+    const int chunks = p.splits;
     const int64_t waves = static_cast<int64_t>(heads) * chunks;
     hipLaunchKernelGGL((attention_keys_kernel<true>), dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), 0, stream,
                        static_cast<const _Float16*>(q), static_cast<const _Float16*>(kc), static_cast<const _Float16*>(vc),
@@ -1042,7 +1559,7 @@ LayerStatus forward_layer(const qmm_layer_config& cfg, const qmm_layer_weights& 
     const size_t o_norm = take(S * hid * 2), o_q = take(S * qd * 2), o_k = take(S * kvd * 2), o_v = take(S * kvd * 2);
     const size_t o_qr = take(S * qd * 2), o_att = take(S * qd * 2), o_proj = take(S * hid * 2), o_h = take(S * hid * 2);
     const size_t o_g = take(S * inter * 2), o_u = take(S * inter * 2), o_act = take(S * inter * 2);
-    const size_t o_down = take(S * hid * 2), o_part = take(attn_part_bytes(seq_len, H, D, kv_len));
+    const size_t o_down = take(S * hid * 2), o_part = take(attn_plan(seq_len, kv_len, H, KVH, D, pos_offset, true, attn_aligned(kc, vc, nullptr), true).bytes);
     char* ws = nullptr;
     hipError_t e = layer_workspace(stream, off, &ws);
     if (e != hipSuccess) return {QMM_ERR_HIP, std::string("layer workspace: ") + hipGetErrorString(e)};
@@ -1139,7 +1656,7 @@ LayerStatus forward_layer(const qmm_layer_config& cfg, const qmm_layer_weights& 
                              pos_offset, cfg.rope_freq_base, cfg.rope_neox != 0, stream)) != hipSuccess)
             return fail(e, "rope");
         e = launch_attention(ws + o_qr, kc, vc, ws + o_att, ws + o_part, seq_len, kv_len, H, KVH, D, pos_offset, scale, true,
-                             stream);
+                             true, stream);
     }
     if (e != hipSuccess) return fail(e, "attention");
     // 5. output projection

@@ -1,0 +1,80 @@
+"""Attention with its keys split over workgroups, and the 16-row matrix-core kernel of short calls.
+
+Against the CPU restatement (oracle/layer_oracle.py).  Both sides round to fp16 once (half an ulp each,
+2^-11 of the largest output together twice that); the 128-row kernel also rounds each weight p to fp16,
+at most 2^-11 sum(p |v|) / sum(p) <= 2^-11 max |v|.  fp32 sums of up to a few thousand terms add 1e-5 max |v|.
+"""
+
+import numpy as np
+import pytest
+
+import layer_oracle as L
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(dev, Q, K, V, start, causal):
+    import torch
+    import qmm
+    q_len, heads, d = Q.shape
+    kv_len, kvh, _ = K.shape
+    t = [torch.from_numpy(x).to(dev) for x in (Q, K, V)]
+    out = torch.full((q_len, heads, d), 7.0, dtype=torch.float16, device=dev)
+    qmm.check(qmm.lib().qmm_gqa_attention(t[0].data_ptr(), t[1].data_ptr(), t[2].data_ptr(), out.data_ptr(), q_len, kv_len, heads,
+                                          kvh, d, start, 0.0, int(causal), torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+def _inputs(q_len, kv_len, heads, kvh, d, seed):
+    r = np.random.default_rng(seed)
+    return [r.standard_normal(s).astype(np.float16) for s in ((q_len, heads, d), (kv_len, kvh, d), (kv_len, kvh, d))]
+
+
+# 16-row tiles: one row to several tiles, 32-key blocks, 128-key ranges and their edges, groups that do
+# not divide the tile, start positions past the keys; 128-row tiles: ranges of two 64-key tiles and more,
+# rows that see no key of their tile's last range.
+@pytest.mark.parametrize("q_len,kv_len,start,heads,kvh,d,causal", [
+    (1, 1, 0, 4, 4, 128, True), (1, 32, 31, 8, 2, 64, True), (1, 33, 32, 8, 1, 128, True), (1, 128, 127, 32, 8, 128, True),
+    (1, 129, 128, 32, 8, 128, True), (1, 4001, 4000, 32, 8, 128, True), (2, 257, 255, 8, 8, 64, True), (3, 500, 497, 21, 3, 128, True),
+    (15, 15, 0, 64, 8, 128, True), (15, 1200, 1185, 8, 1, 64, True), (9, 300, 0, 8, 2, 128, False), (4, 70, 500, 8, 2, 128, True),
+    (5, 40, 0, 8, 2, 128, True), (40, 600, 560, 6, 2, 128, True), (17, 4096, 4079, 20, 4, 64, True),
+    (16, 129, 113, 8, 8, 128, True), (40, 3040, 3000, 32, 8, 128, True), (130, 700, 570, 4, 4, 64, True), (33, 777, 0, 8, 2, 128, False),
+    (257, 257, 0, 4, 4, 128, True), (64, 2048, 100, 16, 2, 64, True)])
+def test_split_attention(cuda, q_len, kv_len, start, heads, kvh, d, causal):
+    Q, K, V = _inputs(q_len, kv_len, heads, kvh, d, 7 * q_len + kv_len + d)
+    got = _run(cuda, Q, K, V, start, causal).astype(np.float32)
+    want = L.gqa_attention(Q, K, V, start, 0.0, causal).astype(np.float32)
+    vmax = float(np.abs(V).max())
+    p16 = q_len >= 16 and 128 % (heads // kvh) == 0
+    bound = 2.0 ** -10 * float(np.abs(want).max()) + (2.0 ** -11 if p16 else 0.0) * vmax + 1e-5 * vmax
+    assert float(np.abs(got - want).max()) <= bound
+
+
+def test_rows_ignore_values_they_do_not_see(cuda):
+    """A later position's infinite or NaN value reaches only the rows that see it."""
+    Q, K, V = _inputs(5, 140, 8, 2, 128, 3)
+    clean = _run(cuda, Q, K, V, 135, True)
+    V[138, 1, 5], V[139, 0, 9] = np.inf, np.nan
+    got = _run(cuda, Q, K, V, 135, True)
+    assert np.array_equal(got[:3].view(np.uint16), clean[:3].view(np.uint16))
+    assert not np.isfinite(got[3:, 4:, 5]).any() and np.isfinite(got[3, :4]).all() and np.isnan(got[4, :4, 9]).all()
+
+
+@pytest.mark.parametrize("off", [0, 1])
+def test_cache_append_alignment(cuda, off):
+    """The new rows reach the cache from 16-byte aligned and from 2-byte aligned sources alike."""
+    import layer
+    import torch
+    import qmm
+    pool = layer.DeviceKVCache(2, 64, 2, 64)  # noqa: F841  (the pool lives as long as the object)
+    Q, K, V = _inputs(20, 20, 4, 2, 64, 11)
+    src = [torch.zeros(K.size + 8, dtype=torch.float16, device=cuda) for _ in range(2)]
+    for s, x in zip(src, (K, V)):
+        s[off:off + x.size] = torch.from_numpy(x.reshape(-1)).to(cuda)
+    q = torch.from_numpy(Q).to(cuda)
+    out = torch.empty_like(q)
+    qmm.check(qmm.lib().qmm_gqa_attention_cached(q.data_ptr(), src[0].data_ptr() + 2 * off, src[1].data_ptr() + 2 * off,
+                                                 out.data_ptr(), 1, 20, 0, 4, 2, 64, 0.0, 1, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy().view(np.uint16), _run(cuda, Q, K, V, 0, True).view(np.uint16))
