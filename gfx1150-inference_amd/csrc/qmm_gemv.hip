@@ -1549,8 +1549,15 @@ hipError_t dispatch_types(int t, const void* A, const Seg* segs, int nseg, int M
     const bool a_vec = (reinterpret_cast<uintptr_t>(A) & 15u) == 0;
     bool fast = a_ok && (t != QMM_TYPE_F16 || K % 16 == 0);
     for (int j = 0; j < nseg; ++j) fast = fast && fast_weights(t, segs[j].W);
-    // the matrix-core GEMV from the format's smallest M (its rows are the same for every M it serves)
-    if (fast && M >= gemv_mfma_min_m(t, identity) && fz.kind == 0 && fz.ea == nullptr && fz.pair == 0) {
+    // the matrix-core GEMV where it serves the matrix at this M; matrices that run different kernels alone
+    // are launched alone
+    int kind = 0;
+    if (fast && fz.kind == 0 && fz.ea == nullptr && fz.pair == 0) {
+        kind = gemv_mfma_kind(t, segs[0].W, M, segs[0].N, K, identity);
+        for (int j = 1; j < nseg; ++j)
+            if (gemv_mfma_kind(t, segs[j].W, M, segs[j].N, K, identity) != kind) return hipErrorNotSupported;
+    }
+    if (kind != 0) {
         const void* W[kMaxSegs];
         void* C[kMaxSegs];
         int N[kMaxSegs];
@@ -1561,7 +1568,7 @@ hipError_t dispatch_types(int t, const void* A, const Seg* segs, int nseg, int M
         }
         const int a_dt = std::is_same<TA, float>::value ? QMM_DTYPE_F32 : QMM_DTYPE_F16;
         const int c_dt = std::is_same<TC, float>::value ? QMM_DTYPE_F32 : QMM_DTYPE_F16;
-        const hipError_t e = launch_gemv_mfma(t, A, a_dt, c_dt, M, K, W, C, N, nseg, stream);
+        const hipError_t e = launch_gemv_mfma(t, A, a_dt, c_dt, M, K, W, C, N, nseg, kind, stream);
         if (e != hipErrorNotSupported) return e;
     }
     if (!fast) {

@@ -1,5 +1,6 @@
 // Small-M GEMV on the matrix cores: C[m, n] = sum_k A[m, k] * dequant(W)[n, k] for the GEMV family's M
-// (16 activation rows per pass), Q4_K and Q6_K weights.
+// (16 activation rows per pass).  Two kernels: the LDS-ring kernel for Q4_K and Q6_K described here, and the
+// register-staged kernel for Q8_0, Q4_0, F16 and other Q6_K rows further below.
 //
 // MI355X design (replaces the reference's wave32 GEMV kernels and their TILE_M = 4 "prefill" variants,
 // src/kernels/dequantize.hip:377-505, 549-685, whose per-row vector work grows with M):
@@ -212,14 +213,13 @@ struct MQ6K {
         p.c2 = 0.0f;
         return p;
     }
-    // B operand of step st: sc (u - 32) for bytes 8 (st & 1) .. + 7 of the lane's slices (weights
-    // j = 8 (st & 1) + 0..7 of group t = st / 2).
-    __device__ static mh8 step(const Raw& r, const Pre& p, int st, uint32_t mg) {
+    // (1024 + u) pairs of step st: bytes 8 (st & 1) .. + 7 of the lane's slices (weights j = 8 (st & 1) + 0..7
+    // of group t = st / 2).
+    __device__ static void codes(const Raw& r, int st, uint32_t mg, uint32_t (&cd)[4]) {
         const int t = st >> 1, jh = st & 1;
         const mu4& q = (t & 1) ? r.lb : r.la;
         const uint32_t L[2] = {jh ? q.z : q.x, jh ? q.w : q.y};
         const uint32_t H[2] = {jh ? r.qh.z : r.qh.x, jh ? r.qh.w : r.qh.y};
-        uint32_t cd[4];
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const uint32_t lo4 = (t < 2 ? L[i] : L[i] >> 4) & 0x0F0F0F0Fu;
@@ -229,6 +229,12 @@ struct MQ6K {
             cd[2 * i] = __builtin_amdgcn_perm(mg, u, 0x07020500u);      // (1024 + u0, 1024 + u2)
             cd[2 * i + 1] = __builtin_amdgcn_perm(mg, u, 0x07030501u);  // (1024 + u1, 1024 + u3)
         }
+    }
+    // B operand of step st: sc (u - 32)
+    __device__ static mh8 step(const Raw& r, const Pre& p, int st, uint32_t mg) {
+        const int t = st >> 1;
+        uint32_t cd[4];
+        codes(r, st, mg, cd);
         // (1024 + u) - 1056 = u - 32 exactly, then times sc: one rounding where |sc (u - 32)| > 2048
         const mh2 off = {static_cast<_Float16>(-1056.0f), static_cast<_Float16>(-1056.0f)};
         const mh2 sv = as_mh2(p.s[t]);
@@ -676,6 +682,379 @@ __global__ __launch_bounds__(64 * kSlots) void gemv_mfma_kernel(const TA* __rest
 }
 
 // ------------------------------------------------------------------------------------------------
+// Block formats, and Q6_K rows that are not whole 16-byte pieces: units staged through registers.
+//
+// K is cut into units of kU k; unit u belongs to slot u % kSlots, one wave each, and the slot sums are added
+// in slot order, so a row's arithmetic depends neither on M nor on the grid.  A wave reads its unit of 16
+// weight rows with 16-byte loads at the rows' own alignment into registers one step ahead, writes them to
+// an LDS area of its own (rows 16-byte aligned, so offsets are constants) and reads the operands back:
+// no barrier but one per batch of row groups.  The activations of a unit go from memory into the operand
+// registers once per window and batch.
+//   * Q8_0: an MFMA step is one 32-weight block, lane quarter c takes its codes 8c..8c+7: v_perm makes
+//     (1024 + u) pairs of u = q + 128, v_pk_add_f16 leaves q exactly, and y += d T in fp32.
+//   * Q4_0: quarter c takes code bytes 4c..4c+3 of the block (k 4c.. and 16 + 4c..); q - 8 is exact.
+//   * F16: the operands as they lie.  Q6_K: below.
+// Bound by the weight stream between a start and an end: 16 waves keep 70 KB of Q8_0 in flight per CU
+// (about 6 TB/s), but first data arrive 4-5 us after the launch and the last wave's unit is worth 2 us.
+// 16 waves of one row group per CU (Q4_0, F16) or two row groups of 8 (Q8_0, Q6_K), whichever measured
+// faster: 8B steps at M = 8, 4 Q8_0 layers, 291 us against 318; 14336 x 4096 Q4_0 13.2 against 17.3.
+// ------------------------------------------------------------------------------------------------
+__device__ __forceinline__ mu4 ld16u(const void* p) {
+    mu4 v;
+    __builtin_memcpy(&v, p, 16);  // any alignment
+    return v;
+}
+
+struct SQ80 {
+    static constexpr int kType = QMM_TYPE_Q8_0, kQK = kQK8_0, kBlockBytes = kBytesQ8_0;
+    static constexpr int kU = 256, kSlots = 8;
+    static constexpr bool kPairs = false, kSplitK = false;
+    __device__ static int k0(int c, int t, int half) { return 32 * t + 8 * c + 4 * half; }
+    // y[r] += d T of the unit's blocks at `u` (4-byte aligned); blocks from nb on are absent
+    __device__ static void unit(const uint8_t* u, int c, int nb, const mh8* a, float* y) {
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(u);
+        const mh2 off = {static_cast<_Float16>(-1152.0f), static_cast<_Float16>(-1152.0f)};
+        const uint32_t mg = mkeep(0x64006400u);
+#pragma unroll
+        for (int b = 0; b < kU / 32; ++b) {
+            // pairs of blocks are 17 dwords: the even block's d and codes start 0 and 2 bytes in, the
+            // odd block's 2 bytes into dword 8 and at dword 9
+            const uint32_t* q = p + 17 * (b >> 1);
+            uint32_t v0, v1, dw;
+            if (b & 1) {
+                v0 = q[9 + 2 * c];
+                v1 = q[10 + 2 * c];
+                dw = q[8] >> 16;
+            } else {
+                const uint32_t w0 = q[2 * c], w1 = q[2 * c + 1], w2 = q[2 * c + 2];
+                v0 = __builtin_amdgcn_alignbyte(w1, w0, 2);
+                v1 = __builtin_amdgcn_alignbyte(w2, w1, 2);
+                dw = q[0];
+            }
+            v0 ^= 0x80808080u;
+            v1 ^= 0x80808080u;
+            const mh2 r0 = as_mh2(__builtin_amdgcn_perm(mg, v0, 0x07010500u)) + off, r1 = as_mh2(__builtin_amdgcn_perm(mg, v0, 0x07030502u)) + off;
+            const mh2 r2 = as_mh2(__builtin_amdgcn_perm(mg, v1, 0x07010500u)) + off, r3 = as_mh2(__builtin_amdgcn_perm(mg, v1, 0x07030502u)) + off;
+            const mh8 bv = {r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
+            const mf4 T = mfma16(a[b], bv, mf4{0.0f, 0.0f, 0.0f, 0.0f});
+            float d = half_bits_to_float(dw);
+            d = b < nb ? d : 0.0f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y[r] = __fmaf_rn(d, T[r], y[r]);
+            if (b & 1) __builtin_amdgcn_sched_barrier(0);  // two blocks' operands in registers at a time
+        }
+    }
+};
+
+struct SQ40 {
+    static constexpr int kType = QMM_TYPE_Q4_0, kQK = kQK4_0, kBlockBytes = kBytesQ4_0;
+    static constexpr int kU = 256, kSlots = 16;
+    static constexpr bool kPairs = true, kSplitK = true;
+    __device__ static int k0(int c, int t, int half) { return 32 * t + 4 * c + 16 * half; }
+    __device__ static void unit(const uint8_t* u, int c, int nb, const mh8* a, float* y) {
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(u);
+        const mh2 lo = {static_cast<_Float16>(-1032.0f), static_cast<_Float16>(-1032.0f)};
+        const mh2 sc = {static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)};
+        const mh2 hi = {static_cast<_Float16>(-72.0f), static_cast<_Float16>(-72.0f)};
+        const uint32_t mg = mkeep(0x64006400u);
+#pragma unroll
+        for (int b = 0; b < kU / 32; ++b) {
+            // pairs of blocks are 9 dwords: the even block's codes start 2 bytes in, the odd block's
+            // d is the upper half of dword 4 and its codes start at dword 5
+            const uint32_t* q = p + 9 * (b >> 1);
+            uint32_t v, dw;
+            if (b & 1) {
+                v = q[5 + c];
+                dw = q[4] >> 16;
+            } else {
+                v = __builtin_amdgcn_alignbyte(q[c + 1], q[c], 2);
+                dw = q[0];
+            }
+            const uint32_t s = v >> 8;
+            const mh2 r0 = as_mh2(andor(v, 0x000F000Fu, mg)) + lo, r1 = as_mh2(andor(s, 0x000F000Fu, mg)) + lo;
+            const mh2 r2 = __builtin_elementwise_fma(as_mh2(andor(v, 0x00F000F0u, mg)), sc, hi);
+            const mh2 r3 = __builtin_elementwise_fma(as_mh2(andor(s, 0x00F000F0u, mg)), sc, hi);
+            const mh8 bv = {r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
+            const mf4 T = mfma16(a[b], bv, mf4{0.0f, 0.0f, 0.0f, 0.0f});
+            float d = half_bits_to_float(dw);
+            d = b < nb ? d : 0.0f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y[r] = __fmaf_rn(d, T[r], y[r]);
+            if (b & 1) __builtin_amdgcn_sched_barrier(0);  // two blocks' operands in registers at a time
+        }
+    }
+};
+
+// rows of whole 16-byte pieces (K % 32 == 0), zeros past a row's end in the last window
+struct SF16 {
+    static constexpr int kType = QMM_TYPE_F16, kQK = 1, kBlockBytes = 2;
+    static constexpr int kU = 128, kSlots = 16;
+    static constexpr bool kPairs = false, kSplitK = false;
+    __device__ static int k0(int c, int t, int half) { return 32 * t + 8 * c + 4 * half; }
+    __device__ static void unit(const uint8_t* u, int c, int, const mh8* a, float* y) {
+        mf4 T = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < kU / 32; ++t) T = mfma16(a[t], *reinterpret_cast<const mh8*>(u + 64 * t + 16 * c), T);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] += T[r];
+    }
+};
+
+// K % 256 == 0: units are whole super-blocks.  The products s (u - 32) of the ring kernel round above 2048; here
+// the sub-scale is cut into s = 16 sh + sl (sh in -8..7, sl in 0..15) and two chains, exact in f16, so a
+// matrix that moves here from v_dot2 loses no precision (one chain: 2.7e-4 against 2.1e-4 in fp16 outputs).
+struct SQ6K {
+    static constexpr int kType = QMM_TYPE_Q6_K, kQK = kQK_K, kBlockBytes = kBytesQ6_K;
+    static constexpr int kU = 256, kSlots = 8;
+    static constexpr bool kPairs = true, kSplitK = false;
+    __device__ static int k0(int c, int t, int half) { return MQ6K::k0(c, t) + 4 * half; }
+    __device__ static void unit(const uint8_t* u, int c, int, const mh8* a, float* y) {
+        const MQ6K::Raw raw = MQ6K::load(u, c);
+        const uint32_t mg = mkeep(0x64006400u);
+        const mh2 off = {static_cast<_Float16>(-1056.0f), static_cast<_Float16>(-1056.0f)};
+        mf4 T = {0.0f, 0.0f, 0.0f, 0.0f}, H = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const int g = t >> 1;  // the lane's group, sub-scale byte h + 2 g of the half's eight
+            const int sc = static_cast<int8_t>((g < 2 ? raw.s0 : raw.s1) >> (8 * ((c & 1) + 2 * (g & 1))));
+            const _Float16 sl = static_cast<_Float16>(static_cast<int16_t>(sc & 15)), sh = static_cast<_Float16>(static_cast<int16_t>(sc >> 4));
+            uint32_t cd[4];
+            MQ6K::codes(raw, t, mg, cd);
+            mh2 lo[4], hi[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const mh2 r = as_mh2(cd[i]) + off;
+                lo[i] = r * mh2{sl, sl};
+                hi[i] = r * mh2{sh, sh};
+            }
+            T = mfma16(a[t], mh8{lo[0][0], lo[0][1], lo[1][0], lo[1][1], lo[2][0], lo[2][1], lo[3][0], lo[3][1]}, T);
+            H = mfma16(a[t], mh8{hi[0][0], hi[0][1], hi[1][0], hi[1][1], hi[2][0], hi[2][1], hi[3][0], hi[3][1]}, H);
+        }
+        const float d = half_bits_to_float(raw.d);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = __fmaf_rn(d, __fmaf_rn(16.0f, H[r], T[r]), y[r]);
+    }
+};
+
+template <class F>
+struct StChunk {
+    static constexpr int kUB = F::kU / F::kQK * F::kBlockBytes;  // bytes of a unit of a row
+    static constexpr int kP = (kUB + 15) / 16;                   // 16-byte pieces of it
+    static constexpr int kRS = 16 * (kP | 1);                    // LDS row stride: odd pieces
+    static constexpr int kBytes = kRows * kRS;                   // one wave's slot
+    static constexpr int kIt = (kRows * kP + 63) / 64;           // pieces per lane
+};
+
+// Activations of one unit for lane (m = row, c): step t's 8 k in the decoder's order; steps at or past kv are
+// zero.
+template <class F>
+struct StAct {
+    static constexpr int S = F::kU / 32;
+    __device__ static __forceinline__ void fp16(const __half* __restrict__ p, int c, int kv, mh8 (&a)[S]) {
+#pragma unroll
+        for (int t = 0; t < S; ++t) {
+            const int k = 32 * t < kv ? 32 * t : 0;
+            mu4 v;
+            if constexpr (F::kSplitK) {
+                uint32_t u[4];
+                __builtin_memcpy(u, p + k + F::k0(c, 0, 0), 8);
+                __builtin_memcpy(u + 2, p + k + F::k0(c, 0, 1), 8);
+                v = mu4{u[0], u[1], u[2], u[3]};
+            } else if constexpr (F::kType == QMM_TYPE_Q6_K) {
+                v = ld16u(p + F::k0(c, t, 0));  // units are whole
+            } else {
+                v = ld16u(p + k + F::k0(c, 0, 0));
+            }
+            __builtin_memcpy(&a[t], &v, 16);
+        }
+#pragma unroll
+        for (int t = 0; t < S; ++t) {
+            if (F::kPairs) {
+                mu4 v;
+                __builtin_memcpy(&v, &a[t], 16);
+                a[t] = pair_order(v);
+            }
+            if (32 * t >= kv) a[t] = mh8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+    }
+    // fp32: scaled by 2^-e (e of the row's unit, returned) and rounded to f16; read twice, for the row
+    // unit's maximum and for its values
+    __device__ static __forceinline__ int fp32(const float* __restrict__ p, int c, int kv, mh8 (&a)[S]) {
+        float mx = 0.0f;
+#pragma unroll
+        for (int t = 0; t < S; ++t)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (32 * t < kv) {
+                    const mu4 v = ld16u(p + F::k0(c, t, h));
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) mx = fmaxf(mx, fabsf(__uint_as_float(v[i])));
+                }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const int e = win_exp(__float_as_uint(mx));
+        __asm__ volatile("" ::: "memory");  // the second read is a read: no values kept over the maximum
+#pragma unroll
+        for (int t = 0; t < S; ++t) {
+            _Float16 x[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            if (32 * t < kv) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const mu4 v = ld16u(p + F::k0(c, t, h));
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[4 * h + i] = static_cast<_Float16>(__builtin_ldexpf(__uint_as_float(v[i]), -e));
+                }
+            }
+            a[t] = F::kPairs ? mh8{x[0], x[2], x[1], x[3], x[4], x[6], x[5], x[7]} : mh8{x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]};
+        }
+        return e;
+    }
+};
+
+template <class F, typename TA, typename TC>
+__global__ __launch_bounds__(64 * F::kSlots, 4) void gemv_staged_kernel(const TA* __restrict__ A, MSegs<TC> sg, int M, int K, int nrg,
+                                                                     int lrows) {
+    using CK = StChunk<F>;
+    constexpr bool kF32 = std::is_same<TA, float>::value;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, c = lane >> 4;
+    const int m0 = blockIdx.y * lrows;
+    const int mr = min(lrows, M - m0);
+    const int row_bytes = K / F::kQK * F::kBlockBytes;
+    const int nun = (K + F::kU - 1) / F::kU;
+    const int nwin = (nun + F::kSlots - 1) / F::kSlots;
+    const int mine = (nrg - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
+    uint8_t* slot = mlds + w * CK::kBytes;
+    uint8_t* red = mlds + F::kSlots * CK::kBytes;
+    const int qa = (lrows + 3) >> 2, qrows = (mr + 3) >> 2;
+
+    // this lane's pieces of a unit's 16 rows (spare lanes repeat the last): row, byte in the row's unit
+    int prow[CK::kIt], pby[CK::kIt];
+#pragma unroll
+    for (int i = 0; i < CK::kIt; ++i) {
+        const int idx = min(lane + 64 * i, kRows * CK::kP - 1);
+        prow[i] = idx / CK::kP;
+        pby[i] = 16 * (idx - prow[i] * CK::kP);
+    }
+    // The pending request: its loads always run, without branches around them (a merge of loaded and kept
+    // registers would wait for the loads); an absent unit reads the start of its segment.  Rows past the
+    // segment repeat its last row (never stored).  A piece past its row, and one that would run past the
+    // matrix and is read from the matrix's last 16 bytes, are put right when the unit is taken (fix).
+    mu4 st[CK::kIt];
+    int p_rows = 0, p_valid = 0, p_last = 0;
+    bool p_fix = false;
+    auto piece_at = [&](int i) { return min(prow[i], p_rows - 1) * row_bytes + (pby[i] < p_valid ? pby[i] : 0); };
+    auto request = [&](int b, int j) {
+        const int u = F::kSlots * j + w;
+        const bool live = b < mine && u < nun;
+        const int g = static_cast<int>(blockIdx.x) + (live ? b : 0) * static_cast<int>(gridDim.x);
+        const uint8_t* W;
+        TC* Cs;
+        int N, g0;
+        seg_pick(sg, g, W, Cs, N, g0);
+        const int r0 = (g - g0) * kRows, u0 = u * CK::kUB;
+        const int64_t last = static_cast<int64_t>(N - r0) * row_bytes - u0 - 16;  // the matrix's last 16 bytes
+        p_rows = min(kRows, N - r0);
+        p_valid = row_bytes - u0;
+        p_last = static_cast<int>(min(last, int64_t{INT_MAX}));
+        p_fix = live && (p_rows < kRows || p_valid < CK::kUB || (kRows - 1) * row_bytes + 16 * (CK::kP - 1) > p_last);
+        const uint8_t* base = live ? W + static_cast<size_t>(r0) * row_bytes + u0 : sg.W[0];
+        int at[CK::kIt];
+#pragma unroll
+        for (int i = 0; i < CK::kIt; ++i) at[i] = live ? prow[i] * row_bytes + pby[i] : 0;
+        if (p_fix) {
+#pragma unroll
+            for (int i = 0; i < CK::kIt; ++i) at[i] = min(piece_at(i), p_last);
+        }
+#pragma unroll
+        for (int i = 0; i < CK::kIt; ++i) st[i] = ld16u(base + at[i]);
+    };
+    auto fix = [&]() {
+#pragma unroll
+        for (int i = 0; i < CK::kIt; ++i) {
+            const int s = max(piece_at(i) - p_last, 0);
+            const mu4 v = st[i];
+            uint64_t lo = (static_cast<uint64_t>(v.y) << 32) | v.x, hi = (static_cast<uint64_t>(v.w) << 32) | v.z;
+            if (s >= 8) {
+                lo = hi >> (8 * (s - 8));
+                hi = 0;
+            } else if (s > 0) {
+                lo = (lo >> (8 * s)) | (hi << (64 - 8 * s));
+                hi >>= 8 * s;
+            }
+            const bool in = pby[i] < p_valid;
+            st[i] = mu4{in ? static_cast<uint32_t>(lo) : 0u, in ? static_cast<uint32_t>(lo >> 32) : 0u,
+                        in ? static_cast<uint32_t>(hi) : 0u, in ? static_cast<uint32_t>(hi >> 32) : 0u};
+        }
+    };
+    const TA* arow = A + static_cast<size_t>(m0 + (n < mr ? n : 0)) * K;
+    request(0, 0);
+    mh8 a[F::kU / 32];
+    int eo[4] = {0, 0, 0, 0};
+    for (int b0 = 0; b0 < mine; b0 += kBG) {
+        const int bs = min(kBG, mine - b0);
+        for (int j = 0; j < nwin; ++j) {
+            const int kv = K - (F::kSlots * j + w) * F::kU;  // k of this wave's unit and after it (<= 0: no unit)
+            if (kv > 0 && (b0 == 0 || nwin > 1)) {
+                if constexpr (kF32) {
+                    const int e = StAct<F>::fp32(arow + (K - kv), c, kv, a);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) eo[r] = __shfl(e, 4 * c + r, 64);
+                } else {
+                    StAct<F>::fp16(arow + (K - kv), c, kv, a);
+                }
+            }
+#pragma unroll 1
+            for (int q = 0; q < bs; ++q) {
+                if (p_fix) fix();
+                // the slot is this wave's own, and a wave's LDS operations run in order
+#pragma unroll
+                for (int i = 0; i < CK::kIt; ++i) *reinterpret_cast<mu4*>(slot + prow[i] * CK::kRS + pby[i]) = st[i];
+                const bool row_end = q + 1 == bs, win_end = row_end && j + 1 == nwin;
+                request(win_end ? b0 + bs : row_end ? b0 : b0 + q + 1, win_end ? 0 : row_end ? j + 1 : j);
+                if (kv > 0) {
+                    const uint8_t* ub = slot + n * CK::kRS;
+                    float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                    F::unit(ub, c, kv / 32, a, y);
+                    // the wave's slot partial of this row group: unit after unit, in place
+                    mf4* acc = reinterpret_cast<mf4*>(red + ((q * F::kSlots + w) * 16 * qa + lane) * 16);
+                    if (c < qrows) {
+                        mf4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+                        if (j > 0) v = *acc;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) v[r] += kF32 && eo[r] != 0 ? __builtin_ldexpf(y[r], eo[r]) : y[r];
+                        *acc = v;
+                    }
+                }
+            }
+        }
+        // end of the batch: wave v adds row group v's slot partials in slot order (slots without units: none)
+        lds_sync();
+        const int slots = min(nun, F::kSlots);
+        if (w < bs && c < qrows) {
+            const uint8_t* rp = red + (w * F::kSlots * 16 * qa + lane) * 16;
+            mf4 sum = *reinterpret_cast<const mf4*>(rp);
+            for (int s = 1; s < slots; ++s) sum += *reinterpret_cast<const mf4*>(rp + s * 256 * qa);
+            const int g = static_cast<int>(blockIdx.x) + (b0 + w) * static_cast<int>(gridDim.x);
+            const uint8_t* W;
+            TC* Cp;
+            int N, g0;
+            seg_pick(sg, g, W, Cp, N, g0);
+            const int row = (g - g0) * kRows + n;
+            if (row < N) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int m = 4 * c + r;
+                    if (m < mr) mstore<TC>(Cp + static_cast<size_t>(m0 + m) * N + row, sum[r]);
+                }
+            }
+        }
+        if (b0 + kBG < mine) lds_sync();  // the partials are free again
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
 // Host side.
 // ------------------------------------------------------------------------------------------------
 std::mutex g_mm_mutex;
@@ -707,7 +1086,7 @@ hipError_t mdev(MDev& out) {
     return hipSuccess;
 }
 
-hipError_t mocc(const void* kern, size_t lds, int& blocks) {
+hipError_t mocc(const void* kern, int threads, size_t lds, int& blocks) {
     static std::unordered_map<std::string, int> cache;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -733,7 +1112,7 @@ hipError_t mocc(const void* kern, size_t lds, int& blocks) {
         if (e != hipSuccess) return e;
     }
     int nb = 0;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, 64 * kSlots, lds);
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, threads, lds);
     if (e != hipSuccess) return e;
     blocks = nb > 0 ? nb : 1;
     cache[key] = blocks;
@@ -795,17 +1174,17 @@ hipError_t mlaunch_ring(const void* A, const MSegs<TC>& sg, int nrg, int M, int 
     if (p3.rows == 0) return hipErrorNotSupported;
     hipError_t e;
     int occ3 = 0, occ4 = 0;
-    if ((e = mocc(mkern<F, R, 3, TA, TC>(), mlds_bytes<F, TA>(p3.rows, 3, p3.bg), occ3)) != hipSuccess) return e;
+    if ((e = mocc(mkern<F, R, 3, TA, TC>(), 64 * kSlots, mlds_bytes<F, TA>(p3.rows, 3, p3.bg), occ3)) != hipSuccess) return e;
     bool use4 = false;
     if (p4.rows > 0) {
-        if ((e = mocc(mkern<F, R, 4, TA, TC>(), mlds_bytes<F, TA>(p4.rows, 4, p4.bg), occ4)) != hipSuccess) return e;
+        if ((e = mocc(mkern<F, R, 4, TA, TC>(), 64 * kSlots, mlds_bytes<F, TA>(p4.rows, 4, p4.bg), occ4)) != hipSuccess) return e;
         use4 = p4.passes < p3.passes || (p4.passes == p3.passes && p4.bg >= p3.bg && 3 * occ4 > 2 * occ3);
     }
     if constexpr (F::kType == QMM_TYPE_Q6_K) {
         const MPlan p2 = mplan<F, TA>(M, 2, di.max_lds);  // (its rows per pass at most p3's)
         int occ2 = 0;
         if (p2.rows > 0 && p2.passes <= p3.passes) {
-            if ((e = mocc(mkern<F, R, 2, TA, TC>(), mlds_bytes<F, TA>(p2.rows, 2, p2.bg), occ2)) != hipSuccess) return e;
+            if ((e = mocc(mkern<F, R, 2, TA, TC>(), 64 * kSlots, mlds_bytes<F, TA>(p2.rows, 2, p2.bg), occ2)) != hipSuccess) return e;
             if (occ2 > occ3 && occ2 > occ4) return mlaunch<F, R, 2, TA, TC>(A, sg, nrg, M, K, a_vec, p2, occ2, di.cus, stream);
         }
     }
@@ -844,6 +1223,48 @@ hipError_t mdispatch(const void* A, const void* const* W, void* const* C, const 
     return mlaunch_ring<F, 4, TA, TC>(A, sg, nrg, M, K, a_vec, di, stream);
 }
 
+// Passes of up to 16 activation rows, balanced.
+template <class F, typename TA, typename TC>
+hipError_t staged_dispatch(const void* A, const void* const* W, void* const* C, const int* N, int count, int M, int K,
+                           hipStream_t stream) {
+    using CK = StChunk<F>;
+    MSegs<TC> sg;
+    int nrg = 0;
+    for (int j = 0; j < 4; ++j) {
+        const int s = j < count ? j : 0;
+        sg.W[j] = static_cast<const uint8_t*>(W[s]);
+        sg.C[j] = static_cast<TC*>(C[s]);
+        sg.N[j] = N[s];
+        if (j < count) nrg += (N[j] + kRows - 1) / kRows;
+        sg.gend[j] = j < count ? nrg : INT_MAX;
+    }
+    MDev di;
+    hipError_t e = mdev(di);
+    if (e != hipSuccess) return e;
+    const int passes = (M + kMRows - 1) / kMRows;
+    if (passes > 65535) return hipErrorNotSupported;
+    const int lrows = (M + passes - 1) / passes;
+    const size_t lds = F::kSlots * (CK::kBytes + kBG * 256 * static_cast<size_t>((lrows + 3) / 4));
+    const void* kern = reinterpret_cast<const void*>(&gemv_staged_kernel<F, TA, TC>);
+    int occ = 0;
+    if ((e = mocc(kern, 64 * F::kSlots, lds, occ)) != hipSuccess) return e;
+    const dim3 grid(min(nrg, max(1, occ * di.cus)), passes);
+    hipLaunchKernelGGL((gemv_staged_kernel<F, TA, TC>), grid, dim3(64 * F::kSlots), lds, stream, static_cast<const TA*>(A), sg, M, K, nrg,
+                       lrows);
+    return hipGetLastError();
+}
+
+template <class F>
+hipError_t staged_dtypes(int a_dtype, int c_dtype, const void* A, const void* const* W, void* const* C, const int* N, int count,
+                         int M, int K, hipStream_t stream) {
+    if (a_dtype == QMM_DTYPE_F32) {
+        if (c_dtype == QMM_DTYPE_F32) return staged_dispatch<F, float, float>(A, W, C, N, count, M, K, stream);
+        return staged_dispatch<F, float, __half>(A, W, C, N, count, M, K, stream);
+    }
+    if (c_dtype == QMM_DTYPE_F32) return staged_dispatch<F, __half, float>(A, W, C, N, count, M, K, stream);
+    return staged_dispatch<F, __half, __half>(A, W, C, N, count, M, K, stream);
+}
+
 template <class F>
 hipError_t mdtypes(int a_dtype, int c_dtype, const void* A, const void* const* W, void* const* C, const int* N, int count,
                    int M, int K, hipStream_t stream) {
@@ -857,24 +1278,50 @@ hipError_t mdtypes(int a_dtype, int c_dtype, const void* A, const void* const* W
 
 }  // namespace
 
-// Where the matrix-core GEMV runs.  Q4_K: from M = 2 (the v_dot2 GEMV is faster at M = 1; 70B gate
-// 28672 x 8192: 26 against 30 us), and at M = 1 too in row-identity mode.  Q6_K: from M = 3 (70B down
-// 8192 x 28672: 49-52 us at M = 3, 4 and 55-58 us at M = 8..16 against 41, 42, 72 and 98 us for v_dot2
-// at M = 1, 2, 4, 8: its decode takes about 1.5 times the VALU work of Q4_K); row-identity mode keeps
-// Q6_K on v_dot2 for every M, so that its M = 1 calls (decode) keep the faster kernel.
-int gemv_mfma_min_m(int ggml_type, bool identity) {
-    if (ggml_type == QMM_TYPE_Q4_K) return identity ? 1 : 2;
-    if (ggml_type == QMM_TYPE_Q6_K) return identity ? INT_MAX : 3;
-    return INT_MAX;
+// Which kernel serves a matrix.  The choice depends on the matrix and M alone, never on what shares its
+// launch.
+//   Ring kernel.  Q4_K: from M = 2 (v_dot2 is faster at M = 1; 70B gate 28672 x 8192: 26 against 30 us),
+//   and at M = 1 too in row-identity mode.  Q6_K of whole 16-byte rows: from M = 3 (70B down 8192 x 28672:
+//   49-52 us at M = 3, 4 and 55-58 us at M = 8..16 against 41, 42, 72 and 98 us for v_dot2 at M = 1, 2, 4, 8:
+//   its decode takes about 1.5 times the VALU work of Q4_K).
+//   Staged kernel, from 1024 rows on (below, 16-row groups leave most CUs idle and v_dot2's items of one or
+//   two rows are faster at every M).  us against v_dot2, fp16 activations, weights from memory:
+//     Q8_0  4096 x 4096    M = 4: 8.4 / 7.8    M = 8: 9.0 / 11.8   M = 16: 10.3 / 17.2
+//           14336 x 4096   M = 3: 18.8 / 20.1  M = 8: 19.8 / 30.3  M = 16: 22.1 / 45.7
+//     Q4_0  4096 x 4096    M = 4: 8.2 / 6.5    M = 8: 9.4 / 9.8    M = 16: 11.9 / 14.4
+//           14336 x 4096   M = 3: 12.2 / 15.6  M = 8: 13.2 / 25.3  M = 16: 15.8 / 39.9
+//     F16   4096 x 4096    M = 2: 10.3 / 10.6  M = 8: 11.0 / 17.2  M = 16: 11.9 / 27.0
+//           14336 x 4096   M = 3: 23.6 / 35.6  M = 8: 23.8 / 55.9  M = 16: 24.6 / 76.3
+//     Q6_K  4096 x 14080   M = 4: 19.6 / 20.0  M = 8: 19.5 / 30.3  M = 16: 23.8 / 55.3
+//   so F16 from M = 3; the others from M = 5, Q8_0 and Q4_0 from M = 3 where the weights, not the launch, set
+//   the time (2^25 of them; Q4_0 with 8192 rows and more, which fill the CUs).
+// Row-identity mode keeps every format but Q4_K on v_dot2 for every M, so that M = 1 calls (decode) keep the
+// faster kernel.
+int gemv_mfma_kind(int ggml_type, const void* W, int M, int N, int K, bool identity) {
+    const uintptr_t wa = reinterpret_cast<uintptr_t>(W);
+    if (N < 1 || K < 1) return 0;
+    // ring kernel: chunks are copied in 16-byte pieces, so rows must be whole pieces
+    if (ggml_type == QMM_TYPE_Q4_K) return M >= (identity ? 1 : 2) && wa % 16 == 0 && K % 256 == 0 ? 1 : 0;
+    if (identity || M < 3) return 0;
+    if (ggml_type == QMM_TYPE_Q6_K && wa % 16 == 0 && K % 2048 == 0) return 1;
+    if (N < 1024 || wa % 2 != 0 || K % (ggml_type == QMM_TYPE_Q6_K ? 256 : 32) != 0) return 0;
+    const bool large = static_cast<int64_t>(N) * K >= int64_t{1} << 25;
+    const bool early = ggml_type == QMM_TYPE_F16 || (large && (ggml_type == QMM_TYPE_Q8_0 || (ggml_type == QMM_TYPE_Q4_0 && N >= 8192)));
+    return M >= (early ? 3 : 5) ? 2 : 0;
 }
 
 hipError_t launch_gemv_mfma(int ggml_type, const void* A, int a_dtype, int c_dtype, int M, int K, const void* const* W,
-                            void* const* C, const int* N, int count, hipStream_t stream) {
-    if (count < 1 || count > 4 || M < 1 || K < 256 || K % 256 != 0) return hipErrorNotSupported;
-    for (int j = 0; j < count; ++j)
-        if (N[j] < 1 || (reinterpret_cast<uintptr_t>(W[j]) & 15u) != 0) return hipErrorNotSupported;
-    // the weight chunks are copied in 16-byte pieces: rows must be whole pieces
-    if (ggml_type == QMM_TYPE_Q6_K && K % 2048 != 0) return hipErrorNotSupported;
+                            void* const* C, const int* N, int count, int kind, hipStream_t stream) {
+    if (count < 1 || count > 4 || M < 1) return hipErrorNotSupported;
+    if (kind == 2) {
+        switch (ggml_type) {
+            case QMM_TYPE_Q8_0: return staged_dtypes<SQ80>(a_dtype, c_dtype, A, W, C, N, count, M, K, stream);
+            case QMM_TYPE_Q4_0: return staged_dtypes<SQ40>(a_dtype, c_dtype, A, W, C, N, count, M, K, stream);
+            case QMM_TYPE_F16: return staged_dtypes<SF16>(a_dtype, c_dtype, A, W, C, N, count, M, K, stream);
+            case QMM_TYPE_Q6_K: return staged_dtypes<SQ6K>(a_dtype, c_dtype, A, W, C, N, count, M, K, stream);
+            default: return hipErrorNotSupported;
+        }
+    }
     switch (ggml_type) {
         case QMM_TYPE_Q4_K: return mdtypes<MQ4K>(a_dtype, c_dtype, A, W, C, N, count, M, K, stream);
         case QMM_TYPE_Q6_K: return mdtypes<MQ6K>(a_dtype, c_dtype, A, W, C, N, count, M, K, stream);

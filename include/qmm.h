@@ -65,13 +65,17 @@ size_t qmm_weight_bytes(int ggml_type, int64_t n, int64_t k);
 /* C[M,N] (c_dtype) = A[M,K] (a_dtype) @ dequant(W)[N,K]^T with fp32 accumulation.
  * M < qmm_gemv_max_m() (17) runs the bandwidth-bound GEMV kernels; larger M runs the f16-MFMA
  * prefill GEMM (a 32-row tile up to M = 32), whose rows agree with the M = 1 call within the
- * prefill accuracy bound.  Among GEMV sizes each format takes the faster of two kernel families:
- * Q4_K the matrix-core GEMV from M = 2, Q6_K from M = 3 (16-byte aligned weights, K a multiple of
- * 2048), and the v_dot2 GEMV below that and for the other formats.  Rows are bit-identical for
- * every M within one family, and the two families agree within the GEMV accuracy bound.  With
- * qmm_set_row_identity(1) every GEMV-size M runs one family (Q4_K the matrix-core GEMV, the other
- * formats the v_dot2 GEMV), so that every row is bit-identical to the M = 1 call, as in the
- * reference.
+ * prefill accuracy bound.  Among GEMV sizes each matrix takes the faster of two kernel families, by
+ * its type, rows and size and by M alone:
+ *   v_dot2 GEMV       every M below the following;
+ *   matrix-core GEMV  Q4_K (16-byte aligned) from M = 2; Q6_K from M = 3 where K is a multiple of 2048 and
+ *                     the weights are 16-byte aligned, else from M = 5; F16 from M = 3; Q8_0 and Q4_0 from
+ *                     M = 5, or from M = 3 with 2^25 weights and more (Q4_0: and 8192 rows).  All but Q4_K
+ *                     and the first Q6_K case: matrices of 1024 rows and more, K a multiple of 32.
+ * Rows are bit-identical for every M within one family, and the two families agree within the GEMV
+ * accuracy bound.  With qmm_set_row_identity(1) every GEMV-size M runs one family (Q4_K the
+ * matrix-core GEMV, the other formats the v_dot2 GEMV), so that every row is bit-identical to the
+ * M = 1 call, as in the reference.
  * Generalises launch_matmul_q{4_0,8_0,4_k,6_k}_device (reference
  * src/kernels/dequantize.h:98-132, dispatch at dequantize.hip:778/896/1014/1132). */
 int qmm_gemm(int ggml_type, const void* A, int a_dtype, const void* W, void* C, int c_dtype,
@@ -160,8 +164,7 @@ int qmm_set_thread_gemv_max_m(int m);
  * With 1, qmm_gemm, qmm_gemm_noalloc and qmm_gemm_batch run every M < qmm_gemv_max_m() of a
  * format on one kernel family, so that rows match the M = 1 call bit for bit: Q4_K on the
  * matrix-core GEMV (its M = 1 a few microseconds slower than the v_dot2 GEMV on large matrices),
- * Q6_K and the other formats on the v_dot2 GEMV (Q6_K's M >= 3 then slower than the matrix-core
- * GEMV).  The reference-API launchers (qmm_matmul_q*_device / _host) always run in this mode. */
+ * Q6_K and the other formats on the v_dot2 GEMV (slower than the matrix-core GEMV at the larger M).  The reference-API launchers (qmm_matmul_q*_device / _host) always run in this mode. */
 int qmm_set_row_identity(int on);
 int qmm_row_identity(void);
 
