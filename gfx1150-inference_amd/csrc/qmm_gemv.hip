@@ -681,6 +681,10 @@ __device__ __forceinline__ void mac_window(const typename F::Raw (&cur)[YT], int
 // thread's items (16 consecutive activations each, at most kFuseOwn) is issued first (A, R and
 // the norm weights, 16-byte vectors), then v is formed, v^2 is reduced over the workgroup for the
 // norm kinds, and the staged fp16 pairs and sums are written as StageItem::store does.
+// A lane's vectors lie 32 or 64 bytes apart, so each load instruction takes the address unit 32 to 64
+// cycles: only the waves that hold items load (K = 4096 has items for 4 of 8 waves), and the loads go out
+// before the first weights, which return behind them.  8B decode q/k/v 13.1 -> 7.4 us, gate/up 21.3 ->
+// 16.5 us against loads by every thread for both of its places, behind the weights.
 constexpr int kFuseOwn = 2;
 // The folded staging exists for one fp16 activation row (decode) and where its registers fit
 // beside the kernel's own (1024-thread workgroups have 128 per lane: one row per item there,
@@ -690,92 +694,106 @@ constexpr bool kFoldable = MR == 1 && std::is_same<TA, __half>::value && (NW <= 
 typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
 
 template <class F, int MR, int NW>
-__device__ __forceinline__ void stage_fused(const __half* A, const GemvFuse& fz, int M, int K, int m0, int nwin, int tid) {
+struct FusedStage {
     static_assert(MR == 1, "one activation row");
-    __shared__ float red[NW];
-    const int items = nwin * 256;
-    const _Float16* a16 = reinterpret_cast<const _Float16*>(A) + static_cast<size_t>(m0) * K;
-    const _Float16* r16 = static_cast<const _Float16*>(fz.R) + static_cast<size_t>(m0) * K;
-    const bool two = fz.kind == 2;
-    h16x8 av[kFuseOwn][2], rv[kFuseOwn][2], wv[kFuseOwn][2];
+    h16x8 av[kFuseOwn][2], rv[kFuseOwn][2];
+    u32x4 wv[kFuseOwn][4];  // 16 norm weights: F32, or F16 in the first two
     int kk[kFuseOwn];
+
+    __device__ __forceinline__ void load(const __half* A, const GemvFuse& fz, int M, int K, int m0, int nwin, int tid) {
+        const int items = nwin * 256;
+        const _Float16* a16 = reinterpret_cast<const _Float16*>(A) + static_cast<size_t>(m0) * K;
+        const _Float16* r16 = static_cast<const _Float16*>(fz.R) + static_cast<size_t>(m0) * K;
+        const int wave0 = __builtin_amdgcn_readfirstlane(tid & ~63);
 #pragma unroll
-    for (int j = 0; j < kFuseOwn; ++j) {
-        const int it = min(tid + 64 * NW * j, items - 1);
-        const int w = it >> 8, q = (it >> 6) & 3, ln = it & 63;
-        const int k = w * kGemvWindow + F::xk(ln, 2 * q);
-        kk[j] = k;
-        const int off = m0 < M && k < K ? k : 0;
+        for (int j = 0; j < kFuseOwn; ++j) {
+            const int it = min(tid + 64 * NW * j, items - 1);
+            const int w = it >> 8, q = (it >> 6) & 3, ln = it & 63;
+            const int k = w * kGemvWindow + F::xk(ln, 2 * q);
+            kk[j] = k;
+            if (wave0 + 64 * NW * j >= items) continue;  // items are whole waves
+            const int off = m0 < M && k < K ? k : 0;
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-            av[j][hh] = *reinterpret_cast<const h16x8*>(a16 + off + 8 * hh);
-            if (two) rv[j][hh] = *reinterpret_cast<const h16x8*>(r16 + off + 8 * hh);
-            {
-                if (fz.w_f32) {  // an F32 norm weight is rounded to f16 first, as the reference's host does
-                    const float* wf = static_cast<const float*>(fz.w) + off + 8 * hh;
-                    const float4 lo = *reinterpret_cast<const float4*>(wf), hi = *reinterpret_cast<const float4*>(wf + 4);
-                    wv[j][hh] = h16x8{static_cast<_Float16>(lo.x), static_cast<_Float16>(lo.y), static_cast<_Float16>(lo.z),
-                                      static_cast<_Float16>(lo.w), static_cast<_Float16>(hi.x), static_cast<_Float16>(hi.y),
-                                      static_cast<_Float16>(hi.z), static_cast<_Float16>(hi.w)};
-                } else {
-                    wv[j][hh] = *reinterpret_cast<const h16x8*>(static_cast<const _Float16*>(fz.w) + off + 8 * hh);
-                }
+            for (int hh = 0; hh < 2; ++hh) av[j][hh] = *reinterpret_cast<const h16x8*>(a16 + off + 8 * hh);
+            if (fz.kind == 2) {
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) rv[j][hh] = *reinterpret_cast<const h16x8*>(r16 + off + 8 * hh);
+            }
+            const u32x4* wp = reinterpret_cast<const u32x4*>(static_cast<const char*>(fz.w) + static_cast<size_t>(off) * (fz.w_f32 ? 4 : 2));
+#pragma unroll
+            for (int i = 0; i < 2; ++i) wv[j][i] = wp[i];
+            if (fz.w_f32) {
+#pragma unroll
+                for (int i = 2; i < 4; ++i) wv[j][i] = wp[i];
             }
         }
     }
-    float ss = 0.0f;
-#pragma unroll
-    for (int j = 0; j < kFuseOwn; ++j) {
-        const bool ok = tid + 64 * NW * j < items && m0 < M && kk[j] < K;
-#pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-            h16x8 v = av[j][hh];
-            if (two) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    v[e] = static_cast<_Float16>(static_cast<float>(v[e]) + static_cast<float>(rv[j][hh][e]));
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                v[e] = ok ? v[e] : static_cast<_Float16>(0.0f);
-                const float f = static_cast<float>(v[e]);
-                ss += f * f;
-            }
-            av[j][hh] = v;
-        }
+
+    // norm weight e of vector hh of item j; an F32 weight is rounded to f16 first, as the reference's host does
+    __device__ __forceinline__ float weight(const GemvFuse& fz, int j, int hh, int e) const {
+        if (fz.w_f32) return static_cast<float>(static_cast<_Float16>(__uint_as_float(wv[j][2 * hh + (e >> 2)][e & 3])));
+        return half_bits_to_float(wv[j][hh][e >> 1] >> (16 * (e & 1)));
     }
+
+    __device__ __forceinline__ void finish(const GemvFuse& fz, int M, int K, int m0, int nwin, int tid) {
+        __shared__ float red[NW];
+        const int items = nwin * 256;
+        const bool two = fz.kind == 2;
+        float ss = 0.0f;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
-    if ((tid & 63) == 0) red[tid >> 6] = ss;
-    __syncthreads();
-    float t = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NW; ++i) t += red[i];
-    const float scale = rsqrtf(t / static_cast<float>(K) + fz.eps);
-#pragma unroll
-    for (int j = 0; j < kFuseOwn; ++j) {
-        const int it = tid + 64 * NW * j;
-        if (it < items) {
-            uint32_t wd[8];
+        for (int j = 0; j < kFuseOwn; ++j) {
+            if (__builtin_amdgcn_readfirstlane(tid & ~63) + 64 * NW * j >= items) continue;  // nothing loaded
+            const bool ok = m0 < M && kk[j] < K;
 #pragma unroll
             for (int hh = 0; hh < 2; ++hh) {
                 h16x8 v = av[j][hh];
+                if (two) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    v[e] = static_cast<_Float16>(static_cast<float>(v[e]) * scale * static_cast<float>(wv[j][hh][e]));
-                __builtin_memcpy(&wd[4 * hh], &v, 16);
-            }
-            StageItem<F, MR, __half> st;
-            // dwords (x0,x1), (x2,x3) -> (x0,x2), (x1,x3), the staged pair order
+                    for (int e = 0; e < 8; ++e)
+                        v[e] = static_cast<_Float16>(static_cast<float>(v[e]) + static_cast<float>(rv[j][hh][e]));
+                }
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                st.h[2 * c] = __builtin_amdgcn_perm(wd[2 * c + 1], wd[2 * c], 0x05040100u);
-                st.h[2 * c + 1] = __builtin_amdgcn_perm(wd[2 * c + 1], wd[2 * c], 0x07060302u);
+                for (int e = 0; e < 8; ++e) {
+                    v[e] = ok ? v[e] : static_cast<_Float16>(0.0f);
+                    const float f = static_cast<float>(v[e]);
+                    ss += f * f;
+                }
+                av[j][hh] = v;
             }
-            st.store(nwin, it >> 8, it & 255);
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+        if ((tid & 63) == 0) red[tid >> 6] = ss;
+        __syncthreads();
+        float t = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) t += red[i];
+        const float scale = rsqrtf(t / static_cast<float>(K) + fz.eps);
+#pragma unroll
+        for (int j = 0; j < kFuseOwn; ++j) {
+            const int it = tid + 64 * NW * j;
+            if (it < items) {
+                uint32_t wd[8];
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    h16x8 v = av[j][hh];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        v[e] = static_cast<_Float16>(static_cast<float>(v[e]) * scale * weight(fz, j, hh, e));
+                    __builtin_memcpy(&wd[4 * hh], &v, 16);
+                }
+                StageItem<F, MR, __half> st;
+                // dwords (x0,x1), (x2,x3) -> (x0,x2), (x1,x3), the staged pair order
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    st.h[2 * c] = __builtin_amdgcn_perm(wd[2 * c + 1], wd[2 * c], 0x05040100u);
+                    st.h[2 * c + 1] = __builtin_amdgcn_perm(wd[2 * c + 1], wd[2 * c], 0x07060302u);
+                }
+                st.store(nwin, it >> 8, it & 255);
+            }
         }
     }
-}
+};
 
 template <int MR, int YT, typename TC>
 __device__ __forceinline__ void reduce_store(float (&acc)[MR][YT], TC* __restrict__ C, int M, int N, int m0, int row0,
@@ -855,7 +873,7 @@ __device__ __forceinline__ SegRef<TC> seg_of(const GemvSegs<TC>& sg, int g) {
 // has been multiplied (the occupancy of several waves per SIMD covers their latency).  Row and
 // window arithmetic is wave-uniform (scalar).  No barrier after staging.
 // Dynamic LDS: MR * nwin * 9216 bytes.
-template <class F, int MR, int YT, int NW, typename TA, typename TC>
+template <class F, int MR, int YT, int NW, bool FU, typename TA, typename TC>
 __global__ __launch_bounds__(64 * NW)
 void gemv_resident_kernel(const TA* __restrict__ A, GemvSegs<TC> sg, int M, int K, int a_vec, int nrg, GemvFuse fz) {
     constexpr bool kF32 = std::is_same<TA, float>::value;
@@ -902,12 +920,11 @@ void gemv_resident_kernel(const TA* __restrict__ A, GemvSegs<TC> sg, int M, int 
     constexpr int kFirst = 2;  // activation items per thread issued before the weight loads
     const int items = nwin * MR * 256;
     Raw b0[YT];
-    bool fused = false;
-    if constexpr (kFoldable<F, MR, YT, NW, TA>) fused = fz.kind != 0;
-    if (fused) {
-        // weight bytes first, then the activations with their prologue
+    if constexpr (FU) {
+        FusedStage<F, MR, NW> fs;
+        fs.load(A, fz, M, K, m0, nwin, tid);
         load_item(gl, wl, b0); next(gl, wl);
-        if constexpr (kFoldable<F, MR, YT, NW, TA>) stage_fused<F, MR, NW>(A, fz, M, K, m0, nwin, tid);
+        fs.finish(fz, M, K, m0, nwin, tid);
     } else {
         if constexpr (kF32) {
             if (tid < nwin * MR) wmax[tid] = 0u;
@@ -1004,7 +1021,7 @@ __device__ __forceinline__ void wait_vmcnt() {
     __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <class F, int MR, int YT, int NW, int NS, typename TA, typename TC>
+template <class F, int MR, int YT, int NW, int NS, bool FU, typename TA, typename TC>
 __global__ __launch_bounds__(64 * NW)
 void gemv_stream_kernel(const TA* __restrict__ A, GemvSegs<TC> sg, int M, int K, int a_vec, int nrg, GemvFuse fz) {
     using WS = WinSlot<F>;
@@ -1060,10 +1077,10 @@ void gemv_stream_kernel(const TA* __restrict__ A, GemvSegs<TC> sg, int M, int K,
         next(gl, wl);
     }
     const int items = nwin * MR * 256;
-    bool fused = false;
-    if constexpr (kFoldable<F, MR, YT, NW, TA>) fused = fz.kind != 0;
-    if (fused) {
-        if constexpr (kFoldable<F, MR, YT, NW, TA>) stage_fused<F, MR, NW>(A, fz, M, K, m0, nwin, tid);
+    if constexpr (FU) {
+        FusedStage<F, MR, NW> fs;
+        fs.load(A, fz, M, K, m0, nwin, tid);
+        fs.finish(fz, M, K, m0, nwin, tid);
     } else {
         if constexpr (kF32) {
             if (tid < nwin * MR) wmax[tid] = 0u;
@@ -1379,8 +1396,10 @@ int seg_table(const Seg* segs, int nseg, const GemvFuse& fz, GemvSegs<TC>& sg) {
     return nrg;
 }
 
-template <class F, int MR, int YT, int NW, typename TA, typename TC>
-hipError_t launch_fast(const void* A, const Seg* segs, int nseg, int M, int K, bool a_vec, const GemvFuse& fz,
+// FU: the activations are staged with a norm prologue (fz.kind != 0).  An instantiation of its own, so that its
+// registers do not lower the occupancy of the plain launches.
+template <class F, int MR, int YT, int NW, bool FU, typename TA, typename TC>
+hipError_t launch_staged(const void* A, const Seg* segs, int nseg, int M, int K, bool a_vec, const GemvFuse& fz,
                        hipStream_t stream) {
     DevInfo di;
     hipError_t e = device_info(di);
@@ -1390,7 +1409,6 @@ hipError_t launch_fast(const void* A, const Seg* segs, int nseg, int M, int K, b
     const size_t res_lds = static_cast<size_t>(MR) * nwin * kSlotBytes;
     const int threads = 64 * NW;
     const bool folded = fz.kind != 0 || fz.ea != nullptr || fz.pair != 0;
-    if (folded && !kFoldable<F, MR, YT, NW, TA>) return hipErrorNotSupported;
     if (fz.pair && (YT != 2 || MR != 1 || nseg != 2 || segs[0].N != segs[1].N || sizeof(TC) != 2)) return hipErrorNotSupported;
     if (fz.kind != 0 && static_cast<int64_t>(nwin) * MR * 256 > static_cast<int64_t>(kFuseOwn) * threads)
         return hipErrorNotSupported;
@@ -1404,7 +1422,7 @@ hipError_t launch_fast(const void* A, const Seg* segs, int nseg, int M, int K, b
             bool ok = row_bytes % 16 == 0 && st_lds <= di.max_lds && wmax_fits;
             for (int j = 0; j < nseg; ++j) ok = ok && (reinterpret_cast<uintptr_t>(segs[j].W) & 15u) == 0;
             if (!ok) return false;
-            const void* kern = reinterpret_cast<const void*>(&gemv_stream_kernel<F, MR, YT, NW, NS, TA, TC>);
+            const void* kern = reinterpret_cast<const void*>(&gemv_stream_kernel<F, MR, YT, NW, NS, FU, TA, TC>);
             int occ = 0;
             if ((e = occupancy(kern, threads, st_lds, occ)) != hipSuccess) return true;
             GemvSegs<TC> sg;
@@ -1412,7 +1430,7 @@ hipError_t launch_fast(const void* A, const Seg* segs, int nseg, int M, int K, b
             const int need = (nrg + NW - 1) / NW;
             const int fill = max(1, occ * di.cus / mblocks);
             const dim3 grid(min(need, fill), mblocks);
-            hipLaunchKernelGGL((gemv_stream_kernel<F, MR, YT, NW, NS, TA, TC>), grid, dim3(threads), st_lds, stream,
+            hipLaunchKernelGGL((gemv_stream_kernel<F, MR, YT, NW, NS, FU, TA, TC>), grid, dim3(threads), st_lds, stream,
                                static_cast<const TA*>(A), sg, M, K, a_vec ? 1 : 0, nrg, fz);
             e = hipGetLastError();
             return true;
@@ -1426,15 +1444,18 @@ hipError_t launch_fast(const void* A, const Seg* segs, int nseg, int M, int K, b
         if (!lane_slots && try_stream(std::integral_constant<int, kGemvNS>{})) return e;
     }
     if (res_lds <= di.max_lds && wmax_fits) {
-        const void* kern = reinterpret_cast<const void*>(&gemv_resident_kernel<F, MR, YT, NW, TA, TC>);
+        const void* kern = reinterpret_cast<const void*>(&gemv_resident_kernel<F, MR, YT, NW, FU, TA, TC>);
         int occ = 0;
         if ((e = occupancy(kern, threads, res_lds, occ)) != hipSuccess) return e;
+        // Q6_K at M = 1: four waves per SIMD.  Its 80 registers would let six in, which is slower (lm_head
+        // 128256 x 4096: 79 -> 84 us).
+        if constexpr (F::kType == QMM_TYPE_Q6_K && MR == 1) occ = min(occ, max(1, 16 / NW));
         GemvSegs<TC> sg;
         const int nrg = seg_table<TC, YT>(segs, nseg, fz, sg);
         const int need = (nrg + NW - 1) / NW;
         const int fill = max(1, occ * di.cus / mblocks);
         const dim3 grid(min(need, fill), mblocks);
-        hipLaunchKernelGGL((gemv_resident_kernel<F, MR, YT, NW, TA, TC>), grid, dim3(threads), res_lds, stream,
+        hipLaunchKernelGGL((gemv_resident_kernel<F, MR, YT, NW, FU, TA, TC>), grid, dim3(threads), res_lds, stream,
                            static_cast<const TA*>(A), sg, M, K, a_vec ? 1 : 0, nrg, fz);
         return hipGetLastError();
     }
@@ -1450,6 +1471,17 @@ hipError_t launch_fast(const void* A, const Seg* segs, int nseg, int M, int K, b
                        static_cast<const TA*>(A), static_cast<const uint8_t*>(segs[0].W), static_cast<TC*>(segs[0].C),
                        M, N, K, a_vec ? 1 : 0);
     return hipGetLastError();
+}
+
+template <class F, int MR, int YT, int NW, typename TA, typename TC>
+hipError_t launch_fast(const void* A, const Seg* segs, int nseg, int M, int K, bool a_vec, const GemvFuse& fz,
+                       hipStream_t stream) {
+    if constexpr (kFoldable<F, MR, YT, NW, TA>) {
+        if (fz.kind != 0) return launch_staged<F, MR, YT, NW, true, TA, TC>(A, segs, nseg, M, K, a_vec, fz, stream);
+    } else if (fz.kind != 0 || fz.ea != nullptr || fz.pair != 0) {
+        return hipErrorNotSupported;
+    }
+    return launch_staged<F, MR, YT, NW, false, TA, TC>(A, segs, nseg, M, K, a_vec, fz, stream);
 }
 
 template <class F, int NW, typename TA, typename TC>
