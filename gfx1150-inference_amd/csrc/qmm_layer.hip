@@ -712,7 +712,8 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnSplit sp, _Flo
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (c0 + i * sg < nv) {
-                    const float w = __builtin_amdgcn_exp2f(pm[i].x - mn);
+                    // a range of which the row sees no key has l = 0 (and mn may still be -inf)
+                    const float w = pm[i].y == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(pm[i].x - mn);
                     l += pm[i].y * w;
                     acc += po[i] * w;
                 }

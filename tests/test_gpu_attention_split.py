@@ -40,7 +40,9 @@ def _inputs(q_len, kv_len, heads, kvh, d, seed):
     (15, 15, 0, 64, 8, 128, True), (15, 1200, 1185, 8, 1, 64, True), (9, 300, 0, 8, 2, 128, False), (4, 70, 500, 8, 2, 128, True),
     (5, 40, 0, 8, 2, 128, True), (40, 600, 560, 6, 2, 128, True), (17, 4096, 4079, 20, 4, 64, True),
     (16, 129, 113, 8, 8, 128, True), (40, 3040, 3000, 32, 8, 128, True), (130, 700, 570, 4, 4, 64, True), (33, 777, 0, 8, 2, 128, False),
-    (257, 257, 0, 4, 4, 128, True), (64, 2048, 100, 16, 2, 64, True)])
+    (257, 257, 0, 4, 4, 128, True), (64, 2048, 100, 16, 2, 64, True),
+    # ranges that a tile's first rows do not see, merged by a thread group of their own
+    (700, 800, 100, 4, 4, 128, True), (700, 790, 90, 8, 2, 64, True)])
 def test_split_attention(cuda, q_len, kv_len, start, heads, kvh, d, causal):
     Q, K, V = _inputs(q_len, kv_len, heads, kvh, d, 7 * q_len + kv_len + d)
     got = _run(cuda, Q, K, V, start, causal).astype(np.float32)
