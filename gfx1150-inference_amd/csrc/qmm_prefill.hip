@@ -299,32 +299,74 @@ struct PQ6K {
     }
 };
 
-// 32-weight block formats: a step covers blocks k0/32 + b, b < 2H (block b absent when
-// kv <= 32b: load() clamps its address to block 0 and scales() zeroes its scale).  Half U
-// holds blocks 2U (S = 0, 1) and 2U + 1 (S = 2, 3).
+// 32-weight block formats: a step covers blocks k0/32 + b, b < 4 (block b absent when kv <= 32b: scales()
+// zeroes its scale).  Half U holds blocks 2U (S = 0, 1) and 2U + 1 (S = 2, 3).
+//
+// Lanes lie a row apart, so every load instruction keeps the address unit busy for all 64 of them, and the
+// loads of short blocks set the time of these formats.  Lane half h therefore loads the two blocks 2h and
+// 2h + 1 as one run (Q8_0 68 bytes in 5 loads, Q4_0 36 bytes in 3, against 8 loads of each where both halves
+// took a part of every block), and prep() hands the parts over with v_permlane32_swap: swap(a, b) leaves
+// (a's lower lanes, b's lower lanes) and (a's upper, b's upper).  Same fragments as before, bit for bit.
+// 4096 x 14336 at M = 31 / 128 / 777 with fp16 activations: Q8_0 59 / 79 / 240 us and Q4_0 55 / 72 / 233 us
+// with 8 loads; now 47 / 62 / 160 us and 32 / 46 / 134 us.
+// A half of which one block exists (`one`), or none, reads only bytes of blocks that do: what lies past a
+// first block's whole 16-byte pieces comes from a load that ends with the block, put right in prep().
+__device__ __forceinline__ void half_swap(uint32_t& a, uint32_t& b) {
+    const auto sw = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = sw[0];
+    b = sw[1];
+}
+
 template <int H>
 struct PQ80 {
+    static_assert(H == 2, "steps of 128 k");
     static constexpr int kH = H;
     static constexpr int kQK = kQK8_0, kBytes = kBytesQ8_0;
-    struct Raw { u32x4p q[2 * H]; uint32_t d[2 * H]; };
+    // loaded: dwords 0..15 of the run in q, 16 in t; after prep(): block b's codes 16h..16h + 15 in q[b], the
+    // scales of blocks 0, 1 in t and of 2, 3 in d
+    struct Raw { u32x4p q[4]; uint32_t t, d; bool one; };
     struct Sc { h2 a0, a1; };
-    __device__ static void prep(Raw&, int) {}
     __device__ static Raw load(const uint8_t* row, int k0, int h, int kv, int) {
-        const uint8_t* b0 = row + static_cast<size_t>(k0 >> 5) * kBytes;
+        const uint8_t* p = row + static_cast<size_t>(k0 >> 5) * kBytes + (kv > 64 * h ? 2 * kBytes * h : 0);
         Raw r;
-#pragma unroll
-        for (int b = 0; b < 2 * H; ++b) {
-            const uint8_t* bb = kv > 32 * b ? b0 + b * kBytes : b0;
-            r.q[b] = ld16(bb + 2 + 16 * h);
-            r.d[b] = ld2(bb);  // always issued (static load count)
-        }
+        r.one = kv < 64 * h + 64;
+        r.q[0] = ld16(p);
+        r.q[1] = ld16(p + 16);
+        r.q[2] = ld16(p + (r.one ? 18 : 32));
+        r.q[3] = ld16(p + (r.one ? 0 : 48));
+        r.t = ld4(p + (r.one ? 0 : 64));
+        r.d = 0u;
         return r;
+    }
+    __device__ static void prep(Raw& r, int) {
+        // run: d (2 bytes), 32 codes, d, 32 codes: the first block's codes lie 2 bytes off, the second's from
+        // dword 9
+        const uint32_t w8 = r.one ? r.q[2].w >> 16 : r.q[2].x;
+        uint32_t w[17] = {r.q[0].x, r.q[0].y, r.q[0].z, r.q[0].w, r.q[1].x, r.q[1].y, r.q[1].z, r.q[1].w, w8,
+                          r.q[2].y, r.q[2].z, r.q[2].w, r.q[3].x, r.q[3].y, r.q[3].z, r.q[3].w, r.t};
+        uint32_t d = __builtin_amdgcn_perm(w8, w[0], 0x07060100u);  // (d of the first block, of the second)
+        uint32_t a[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a[i] = __builtin_amdgcn_alignbyte(w[i + 1], w[i], 2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            half_swap(a[i], a[4 + i]);        // -> block 0, block 2
+            half_swap(w[9 + i], w[13 + i]);   // -> block 1, block 3
+        }
+        r.q[0] = u32x4p{a[0], a[1], a[2], a[3]};
+        r.q[2] = u32x4p{a[4], a[5], a[6], a[7]};
+        r.q[1] = u32x4p{w[9], w[10], w[11], w[12]};
+        r.q[3] = u32x4p{w[13], w[14], w[15], w[16]};
+        r.t = d;
+        r.d = d;
+        half_swap(r.t, r.d);
     }
     template <int U>
     __device__ static Sc scales(const Raw& r, int, int, int kv) {
+        const uint32_t d = U == 0 ? r.t : r.d;
         Sc s;
-        s.a0 = splat(half_bits_to_float(kv > 64 * U ? r.d[2 * U] : 0u));
-        s.a1 = splat(half_bits_to_float(kv > 64 * U + 32 ? r.d[2 * U + 1] : 0u));
+        s.a0 = splat(half_bits_to_float(kv > 64 * U ? d : 0u));
+        s.a1 = splat(half_bits_to_float(kv > 64 * U + 32 ? d >> 16 : 0u));
         return s;
     }
     template <int U, int S>
@@ -346,28 +388,47 @@ struct PQ80 {
 
 template <int H>
 struct PQ40 {
+    static_assert(H == 2, "steps of 128 k");
     static constexpr int kH = H;
     static constexpr int kQK = kQK4_0, kBytes = kBytesQ4_0;
-    struct Raw { u32x4p q[2 * H]; uint32_t d[2 * H]; };
+    // loaded: dwords 0..7 of the run in q[0], q[1], 8 in t; after prep(): block b's 16 code bytes in q[b], the
+    // scales of blocks 0, 1 in t and of 2, 3 in d.  Lane half h takes the block's low (h = 0, k 0..15) or high
+    // (h = 1, k 16..31) nibbles.
+    struct Raw { u32x4p q[4]; uint32_t t, d; bool one; };
     struct Sc { h2 a0, a1; };
-    // lane half h takes the block's low (h = 0, k 0..15) or high (h = 1, k 16..31) nibbles.
-    __device__ static void prep(Raw&, int) {}
-    __device__ static Raw load(const uint8_t* row, int k0, int, int kv, int) {
-        const uint8_t* b0 = row + static_cast<size_t>(k0 >> 5) * kBytes;
+    __device__ static Raw load(const uint8_t* row, int k0, int h, int kv, int) {
+        const uint8_t* p = row + static_cast<size_t>(k0 >> 5) * kBytes + (kv > 64 * h ? 2 * kBytes * h : 0);
         Raw r;
-#pragma unroll
-        for (int b = 0; b < 2 * H; ++b) {
-            const uint8_t* bb = kv > 32 * b ? b0 + b * kBytes : b0;
-            r.q[b] = ld16(bb + 2);
-            r.d[b] = ld2(bb);  // always issued (static load count)
-        }
+        r.one = kv < 64 * h + 64;
+        r.q[0] = ld16(p);
+        r.q[1] = ld16(p + (r.one ? 2 : 16));
+        r.t = ld4(p + (r.one ? 0 : 32));
+        r.q[2] = r.q[3] = u32x4p{0u, 0u, 0u, 0u};
+        r.d = 0u;
         return r;
+    }
+    __device__ static void prep(Raw& r, int) {
+        const uint32_t w4 = r.one ? r.q[1].w >> 16 : r.q[1].x;
+        const uint32_t w[9] = {r.q[0].x, r.q[0].y, r.q[0].z, r.q[0].w, w4, r.q[1].y, r.q[1].z, r.q[1].w, r.t};
+        r.t = r.d = __builtin_amdgcn_perm(w4, w[0], 0x07060100u);
+        half_swap(r.t, r.d);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t a = __builtin_amdgcn_alignbyte(w[i + 1], w[i], 2), b = a, c = w[5 + i], e = c;
+            half_swap(a, b);
+            half_swap(c, e);
+            r.q[0][i] = a;
+            r.q[1][i] = c;
+            r.q[2][i] = b;
+            r.q[3][i] = e;
+        }
     }
     template <int U>
     __device__ static Sc scales(const Raw& r, int, int, int kv) {
+        const uint32_t d = U == 0 ? r.t : r.d;
         Sc s;
-        s.a0 = splat(half_bits_to_float(kv > 64 * U ? r.d[2 * U] : 0u));
-        s.a1 = splat(half_bits_to_float(kv > 64 * U + 32 ? r.d[2 * U + 1] : 0u));
+        s.a0 = splat(half_bits_to_float(kv > 64 * U ? d : 0u));
+        s.a1 = splat(half_bits_to_float(kv > 64 * U + 32 ? d >> 16 : 0u));
         return s;
     }
     template <int U, int S>
