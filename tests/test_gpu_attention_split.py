@@ -53,6 +53,22 @@ def test_split_attention(cuda, q_len, kv_len, start, heads, kvh, d, causal):
     assert float(np.abs(got - want).max()) <= bound
 
 
+@pytest.mark.parametrize("q_len", [3, 40])
+def test_negative_scale(cuda, q_len):
+    import torch
+    import qmm
+    Q, K, V = _inputs(q_len, 200, 8, 2, 128, 5)
+    t = [torch.from_numpy(x).to(cuda) for x in (Q, K, V)]
+    out = torch.empty_like(t[0])
+    qmm.check(qmm.lib().qmm_gqa_attention(t[0].data_ptr(), t[1].data_ptr(), t[2].data_ptr(), out.data_ptr(), q_len, 200, 8, 2, 128,
+                                          200 - q_len, -0.07, 1, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    want = L.gqa_attention(Q, K, V, 200 - q_len, -0.07, True).astype(np.float32)
+    vmax = float(np.abs(V).max())
+    bound = 2.0 ** -10 * float(np.abs(want).max()) + 2.0 ** -11 * vmax + 1e-5 * vmax
+    assert float(np.abs(out.cpu().numpy().astype(np.float32) - want).max()) <= bound
+
+
 def test_rows_ignore_values_they_do_not_see(cuda):
     """A later position's infinite or NaN value reaches only the rows that see it."""
     Q, K, V = _inputs(5, 140, 8, 2, 128, 3)
