@@ -448,6 +448,95 @@ struct PQ40 {
     }
 };
 
+// The 256 x 256 tile's producers of the same formats, and the same fragments: each lane half loads its part of
+// every block and nothing is exchanged.  With one wave per SIMD the exchange is exposed, and two row blocks per
+// wave share the wait for the loads: a wide Q8_0 / Q4_0 launch of 145 us took 159 us with runs.  load() clamps
+// an absent block's address to block 0.
+template <int H>
+struct PQ80W {
+    static constexpr int kH = H;
+    static constexpr int kQK = kQK8_0, kBytes = kBytesQ8_0;
+    struct Raw { u32x4p q[2 * H]; uint32_t d[2 * H]; };
+    struct Sc { h2 a0, a1; };
+    __device__ static void prep(Raw&, int) {}
+    __device__ static Raw load(const uint8_t* row, int k0, int h, int kv, int) {
+        const uint8_t* b0 = row + static_cast<size_t>(k0 >> 5) * kBytes;
+        Raw r;
+#pragma unroll
+        for (int b = 0; b < 2 * H; ++b) {
+            const uint8_t* bb = kv > 32 * b ? b0 + b * kBytes : b0;
+            r.q[b] = ld16(bb + 2 + 16 * h);
+            r.d[b] = ld2(bb);  // always issued (static load count)
+        }
+        return r;
+    }
+    template <int U>
+    __device__ static Sc scales(const Raw& r, int, int, int kv) {
+        Sc s;
+        s.a0 = splat(half_bits_to_float(kv > 64 * U ? r.d[2 * U] : 0u));
+        s.a1 = splat(half_bits_to_float(kv > 64 * U + 32 ? r.d[2 * U + 1] : 0u));
+        return s;
+    }
+    template <int U, int S>
+    __device__ static void frag(const Raw& r, const Sc& sc, int, uint32_t f[4]) {
+        constexpr int u = S >> 1;
+        const u32x4p q = r.q[2 * U + u];
+        const uint32_t w[2] = {(S & 1) ? q.z : q.x, (S & 1) ? q.w : q.y};
+        const h2 off = splat(1152.0f);  // signed codes enter as 1024 + (q + 128)
+        const h2 a = u ? sc.a1 : sc.a0;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            h2 p, qq;
+            bytes_to_h2(w[j] ^ 0x80808080u, off, p, qq);
+            f[2 * j] = as_u32(p * a);
+            f[2 * j + 1] = as_u32(qq * a);
+        }
+    }
+};
+
+template <int H>
+struct PQ40W {
+    static constexpr int kH = H;
+    static constexpr int kQK = kQK4_0, kBytes = kBytesQ4_0;
+    struct Raw { u32x4p q[2 * H]; uint32_t d[2 * H]; };
+    struct Sc { h2 a0, a1; };
+    // lane half h takes the block's low (h = 0, k 0..15) or high (h = 1, k 16..31) nibbles.
+    __device__ static void prep(Raw&, int) {}
+    __device__ static Raw load(const uint8_t* row, int k0, int, int kv, int) {
+        const uint8_t* b0 = row + static_cast<size_t>(k0 >> 5) * kBytes;
+        Raw r;
+#pragma unroll
+        for (int b = 0; b < 2 * H; ++b) {
+            const uint8_t* bb = kv > 32 * b ? b0 + b * kBytes : b0;
+            r.q[b] = ld16(bb + 2);
+            r.d[b] = ld2(bb);  // always issued (static load count)
+        }
+        return r;
+    }
+    template <int U>
+    __device__ static Sc scales(const Raw& r, int, int, int kv) {
+        Sc s;
+        s.a0 = splat(half_bits_to_float(kv > 64 * U ? r.d[2 * U] : 0u));
+        s.a1 = splat(half_bits_to_float(kv > 64 * U + 32 ? r.d[2 * U + 1] : 0u));
+        return s;
+    }
+    template <int U, int S>
+    __device__ static void frag(const Raw& r, const Sc& sc, int h, uint32_t f[4]) {
+        constexpr int u = S >> 1;
+        const u32x4p q = r.q[2 * U + u];
+        const uint32_t w[2] = {(S & 1) ? q.z : q.x, (S & 1) ? q.w : q.y};
+        const h2 off = splat(1032.0f);  // codes enter as 1024 + q, weight is d (q - 8)
+        const h2 a = u ? sc.a1 : sc.a0;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            h2 p, qq;
+            bytes_to_h2((w[j] >> (4 * h)) & 0x0F0F0F0Fu, off, p, qq);
+            f[2 * j] = as_u32(p * a);
+            f[2 * j + 1] = as_u32(qq * a);
+        }
+    }
+};
+
 // F16 (dense fp16 rows, the operand of the reference's matmul_nt): a lane loads the 8 weights
 // of each of its sub-steps straight into the fragment (natural k order, no conversion).  Needs
 // K % 8 == 0: a chunk is wholly inside K or wholly outside it; one outside reads the row's first
@@ -1612,15 +1701,15 @@ hipError_t launch_p(const void* A, const PfSeg* segs, int nseg, int M, int K, hi
     return launch_grid<P, TC, Tile>(a16, lda, tail_segs, n_tail, M, K, plan.tail_ks, part, rs, stream);
 }
 
-// HN: 64-k halves per step of the 128 x 256 kernel for this format.
-template <template <int> class PF, int HN, typename TA, typename TC>
+// PF: the format's producer, PW: the wide tile's; HN: 64-k halves per step of the 128 x 256 kernel.
+template <template <int> class PF, template <int> class PW, int HN, typename TA, typename TC>
 hipError_t launch_family(const void* A, const PfSeg* segs, int nseg, int M, int K, hipStream_t stream, PfWs* ext) {
     int cus = 0;
     hipError_t e = cu_count(cus);
     if (e != hipSuccess) return e;
     int64_t wide_tiles_n = 0;
     for (int i = 0; i < nseg; ++i) wide_tiles_n += (segs[i].N + kWBN - 1) / kWBN;
-    if (use_wide(M, wide_tiles_n, K, cus)) return launch_p<PF<kWH>, TA, TC, kTileWide>(A, segs, nseg, M, K, stream, ext);
+    if (use_wide(M, wide_tiles_n, K, cus)) return launch_p<PW<kWH>, TA, TC, kTileWide>(A, segs, nseg, M, K, stream, ext);
     if (M <= kSmallMaxM) return launch_p<PF<HN>, TA, TC, kTileSmall>(A, segs, nseg, M, K, stream, ext);
     return launch_p<PF<HN>, TA, TC, kTileStd>(A, segs, nseg, M, K, stream, ext);
 }
@@ -1628,11 +1717,11 @@ hipError_t launch_family(const void* A, const PfSeg* segs, int nseg, int M, int 
 template <typename TA, typename TC>
 hipError_t dispatch_p(int t, const void* A, const PfSeg* segs, int nseg, int M, int K, hipStream_t stream, PfWs* ext) {
     switch (t) {
-        case QMM_TYPE_Q4_K: return launch_family<PQ4K, kHalves, TA, TC>(A, segs, nseg, M, K, stream, ext);
-        case QMM_TYPE_Q6_K: return launch_family<PQ6K, kHalves, TA, TC>(A, segs, nseg, M, K, stream, ext);
-        case QMM_TYPE_Q8_0: return launch_family<PQ80, 2, TA, TC>(A, segs, nseg, M, K, stream, ext);
-        case QMM_TYPE_Q4_0: return launch_family<PQ40, 2, TA, TC>(A, segs, nseg, M, K, stream, ext);
-        case QMM_TYPE_F16: return launch_family<PF16, 2, TA, TC>(A, segs, nseg, M, K, stream, ext);
+        case QMM_TYPE_Q4_K: return launch_family<PQ4K, PQ4K, kHalves, TA, TC>(A, segs, nseg, M, K, stream, ext);
+        case QMM_TYPE_Q6_K: return launch_family<PQ6K, PQ6K, kHalves, TA, TC>(A, segs, nseg, M, K, stream, ext);
+        case QMM_TYPE_Q8_0: return launch_family<PQ80, PQ80W, 2, TA, TC>(A, segs, nseg, M, K, stream, ext);
+        case QMM_TYPE_Q4_0: return launch_family<PQ40, PQ40W, 2, TA, TC>(A, segs, nseg, M, K, stream, ext);
+        case QMM_TYPE_F16: return launch_family<PF16, PF16, 2, TA, TC>(A, segs, nseg, M, K, stream, ext);
         default: return hipErrorInvalidValue;
     }
 }
