@@ -424,18 +424,24 @@ int qmm_gqa_attention(const void* Q, const void* K, const void* V, void* out, in
     if (!Q || !out || (kv_len > 0 && (!K || !V))) return fail(QMM_ERR_INVALID_ARGUMENT, "Q, K, V and Out must be non-null.");
     hipStream_t s = static_cast<hipStream_t>(stream);
     void* part = nullptr;
-    // A call of many rows records no pointer into the per-stream scratch when it is captured (a later,
-    // larger call may free it): its keys are not split then.
+    // A call of many rows (head_dim 64 and 128, aligned operands) records no pointer into the per-stream
+    // scratch when it is captured (a later, larger call may free it): its keys are not split then.  Nor on
+    // hipStreamPerThread, whose threads share one scratch and would wait for each other.
     bool may_split = true;
     if (q_len >= 16) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        may_split = hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
-        if (!may_split) (void)hipGetLastError();
+        if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+            (void)hipGetLastError();
+            may_split = false;
+        } else {
+            may_split = cap == hipStreamCaptureStatusNone && s != hipStreamPerThread;
+        }
     }
     const size_t pb = qmm::attention_workspace_bytes(Q, K, V, q_len, kv_len, num_heads, num_kv_heads, head_dim, start_pos,
                                                      causal != 0, may_split);
     hipError_t e;
-    if (pb > 0 && (e = qmm::layer_scratch(s, pb, &part)) != hipSuccess) return hip_fail(e, "attention workspace");
+    std::unique_lock<std::mutex> held;  // until the merge is enqueued
+    if (pb > 0 && (e = qmm::attention_scratch(s, pb, held, &part)) != hipSuccess) return hip_fail(e, "attention workspace");
     const float sc = scale != 0.0f ? scale : 1.0f / std::sqrt(static_cast<float>(head_dim));
     e = qmm::launch_attention(Q, K, V, out, part, q_len, kv_len, num_heads, num_kv_heads, head_dim, start_pos, sc,
                               causal != 0, may_split, s);

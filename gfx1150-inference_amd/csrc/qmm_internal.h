@@ -8,6 +8,7 @@
 
 #include "qmm.h"
 
+#include <mutex>
 #include <string>
 
 namespace qmm {
@@ -163,7 +164,9 @@ LayerStatus kv_cache_layer(int layer, int start, int q_len, int kv_heads, int he
                            int* max_seq);
 LayerStatus forward_layer(const qmm_layer_config& cfg, const qmm_layer_weights& w, const void* x_in, void* x_out,
                           int layer_idx, int seq_len, int pos_offset, hipStream_t stream);
-hipError_t layer_scratch(hipStream_t stream, size_t bytes, void** out);
+// The attention entry points' scratch of `stream`: the caller keeps `held` until its last launch that uses the
+// buffer is enqueued.
+hipError_t attention_scratch(hipStream_t stream, size_t bytes, std::unique_lock<std::mutex>& held, void** out);
 hipError_t release_layer_workspaces();
 
 }  // namespace qmm
