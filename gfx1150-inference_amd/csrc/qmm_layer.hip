@@ -1331,11 +1331,17 @@ AttnPlan attn_plan(int q_len, int kv_len, int heads, int kv_heads, int head_dim,
     int per = most;
     if (may_split && 2 * wgs <= kAttnFill) {
         const int64_t even = (blocks * kv_heads + kAttnFill - 1) / kAttnFill;
-        per = static_cast<int>(std::min<int64_t>(most, std::max<int64_t>(even, mfma ? 2 : 1)));
+        const int max_splits = static_cast<int>(2 * kAttnFill / wgs);
+        per = static_cast<int>(std::min<int64_t>(most, std::max<int64_t>({even, mfma ? 2 : 1, (most + max_splits - 1) / max_splits})));
     }
     p.splits = (most + per - 1) / per;
     p.kps = per * block;
-    p.bytes = p.splits > 1 ? row_bytes * p.splits : 0;
+    // Room for any call of as many rows and keys or fewer: at most a partial result per row and block, and
+    // (max_splits) 2 kAttnFill row tiles of them.  The plan's own need goes up and down with the context (8192
+    // keys make 64 ranges, 8193 make 33), so a buffer sized by it would grow, and move, after a longer call.
+    if (may_split && kv_len > block)
+        p.bytes = static_cast<size_t>(std::min<int64_t>(static_cast<int64_t>(q_len) * heads * ((kv_len + block - 1) / block),
+                                                        2 * kAttnFill * p.tile_rows)) * (head_dim + 2) * sizeof(float);
     return p;
 }
 

@@ -96,3 +96,45 @@ def test_cache_append_alignment(cuda, off):
                                                  out.data_ptr(), 1, 20, 0, 4, 2, 64, 0.0, 1, torch.cuda.current_stream().cuda_stream))
     torch.cuda.synchronize()
     assert np.array_equal(out.cpu().numpy().view(np.uint16), _run(cuda, Q, K, V, 0, True).view(np.uint16))
+
+
+def test_graphs_of_shorter_contexts_after_the_longest_call(cuda):
+    """One eager call at the longest context is enough for captures at every shorter one: none of them
+    allocates, and replays after further eager calls give the eager results."""
+    import torch
+    import qmm
+    heads, kvh, d, longest = 32, 8, 128, 12000
+    g = torch.Generator(device=cuda)
+    g.manual_seed(3)
+    q = torch.randn((1, heads * d), generator=g, device=cuda).half()
+    k, v = (torch.randn((longest, kvh * d), generator=g, device=cuda).half() for _ in range(2))
+    qmm.check(qmm.lib().qmm_release_workspace())
+    stream = torch.cuda.Stream()
+
+    def call(kv, out):
+        qmm.check(qmm.lib().qmm_gqa_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), 1, kv, heads, kvh, d, kv - 1,
+                                              0.0, 1, stream.cuda_stream))
+    torch.cuda.synchronize()
+    eager, replayed, graphs = {}, {}, {}
+    with torch.cuda.stream(stream):
+        for kv in (longest, 8192, 8193, 6000, 4097, 1000, 129):
+            eager[kv] = torch.empty_like(q)
+            call(kv, eager[kv])
+            if kv == longest:
+                stream.synchronize()
+                free = torch.cuda.mem_get_info()[0]
+    stream.synchronize()
+    assert torch.cuda.mem_get_info()[0] == free
+    for kv in (8192, 8193, 6000, 4097, 1000, 129):
+        replayed[kv], graphs[kv] = torch.zeros_like(q), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graphs[kv], stream=stream):
+            call(kv, replayed[kv])
+    for _ in range(3):
+        for kv, graph in graphs.items():
+            replayed[kv].zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream):
+                graph.replay()
+                call(longest, eager[longest])
+            torch.cuda.synchronize()
+            assert torch.equal(replayed[kv], eager[kv]), kv
