@@ -784,8 +784,8 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnSplit sp, _Flo
 //   * those 8 keys are the k order of the second product's operand, so the weights go straight from
 //     the score registers into O^T += V^T P^T; lane (l, q) loads dims D/16 l .. of its 8 keys' V rows
 //     (16 lanes read one whole row) and v_perm transposes them in registers;
-//   * weights stay at fp32 precision: 2^10 p = hi + lo in f16, two products (the scale keeps lo clear
-//     of f16's subnormals; it cancels against the sum).
+//   * weights enter as 2^10 p = hi + lo in f16, two products (the scale cancels against the sum): 22 bits for
+//     p >= 2^-13 of the range's maximum, an absolute error of 2^-35 of it below, where lo is subnormal or 0.
 // The 4 waves of a workgroup take every fourth 32-key block of its range and are merged through LDS in
 // wave order.  8B decode at context 4000 (16 MB of keys and values): 7.8 us and 4.3 us of merge, against
 // 12.2 us and 13.0 us with one wave per (query head, 64 keys) on the vector ALUs, which reads each
@@ -856,140 +856,152 @@ __global__ __launch_bounds__(64 * kRowsWaves) void attention_rows_kernel(
         if constexpr (kRope) rotate_row<D>(qf, dr, q);
     }
     f32x4 o[D / 16];
+    float m_run, l_run;
+    // One pass over the wave's keys.  kCareful: the products run row by row, with the values that the row does
+    // not see cleared and infinite or NaN ones weighted by p > 0 alone.
+    auto scan = [&](auto careful) {
+        constexpr bool kCareful = decltype(careful)::value;
 #pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) o[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m_run = -INFINITY, l_run = 0.0f;
-
-    for (int kb = k_begin + kRowsKeys * w; kb < k_end; kb += kRowsKeys * kRowsWaves) {
-        // keys past the tile's last read that key; their weights are zero
-        f16x8 kf[2][D / 32];
-        uint32_t vd[8][kVW];  // V slices of keys kb + 16 (j / 4) + 4 q + j % 4
+        for (int dt = 0; dt < D / 16; ++dt) o[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        m_run = -INFINITY;
+        l_run = 0.0f;
+        for (int kb = k_begin + kRowsKeys * w; kb < k_end; kb += kRowsKeys * kRowsWaves) {
+            // keys past the tile's last read that key; their weights are zero
+            f16x8 kf[2][D / 32];
+            uint32_t vd[8][kVW];  // V slices of keys kb + 16 (j / 4) + 4 q + j % 4
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const int k = min(kb + 16 * tt + l, n_keys - 1);
-            const _Float16* kr = kbase + static_cast<size_t>(k) * kv_row + 8 * q;
-            if constexpr (kRope)
-                if (k == start_pos) kr = dr.k_new + static_cast<size_t>(g) * D + 8 * q;
+            for (int tt = 0; tt < 2; ++tt) {
+                const int k = min(kb + 16 * tt + l, n_keys - 1);
+                const _Float16* kr = kbase + static_cast<size_t>(k) * kv_row + 8 * q;
+                if constexpr (kRope)
+                    if (k == start_pos) kr = dr.k_new + static_cast<size_t>(g) * D + 8 * q;
 #pragma unroll
-            for (int db = 0; db < D / 32; ++db) kf[tt][db] = *reinterpret_cast<const f16x8*>(kr + 32 * db);
-        }
+                for (int db = 0; db < D / 32; ++db) kf[tt][db] = *reinterpret_cast<const f16x8*>(kr + 32 * db);
+            }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int k = min(kb + 16 * (j >> 2) + 4 * q + (j & 3), n_keys - 1);
-            const _Float16* vr = vbase + static_cast<size_t>(k) * kv_row;
-            if constexpr (kRope)
-                if (k == start_pos) vr = dr.v_new + static_cast<size_t>(g) * D;
-            __builtin_memcpy(vd[j], __builtin_assume_aligned(vr + D / 16 * l, D / 8), 4 * kVW);
-        }
-        if constexpr (kRope) {
-            if (kb + kRowsKeys > start_pos) {  // the block with the new key
+            for (int j = 0; j < 8; ++j) {
+                const int k = min(kb + 16 * (j >> 2) + 4 * q + (j & 3), n_keys - 1);
+                const _Float16* vr = vbase + static_cast<size_t>(k) * kv_row;
+                if constexpr (kRope)
+                    if (k == start_pos) vr = dr.v_new + static_cast<size_t>(g) * D;
+                __builtin_memcpy(vd[j], __builtin_assume_aligned(vr + D / 16 * l, D / 8), 4 * kVW);
+            }
+            if constexpr (kRope) {
+                if (kb + kRowsKeys > start_pos) {  // the block with the new key
 #pragma unroll
-                for (int tt = 0; tt < 2; ++tt) {
-                    const bool is_new = min(kb + 16 * tt + l, n_keys - 1) == start_pos;
-                    f16x8 rot[D / 32];
+                    for (int tt = 0; tt < 2; ++tt) {
+                        const bool is_new = min(kb + 16 * tt + l, n_keys - 1) == start_pos;
+                        f16x8 rot[D / 32];
 #pragma unroll
-                    for (int db = 0; db < D / 32; ++db) rot[db] = kf[tt][db];
-                    rotate_row<D>(rot, dr, q);
+                        for (int db = 0; db < D / 32; ++db) rot[db] = kf[tt][db];
+                        rotate_row<D>(rot, dr, q);
 #pragma unroll
-                    for (int db = 0; db < D / 32; ++db) kf[tt][db] = is_new ? rot[db] : kf[tt][db];
-                    if (rt == 0 && kb + 16 * tt + l == start_pos) {
-                        _Float16* kw = dr.kc + static_cast<size_t>(start_pos) * kv_row + static_cast<size_t>(g) * D + 8 * q;
+                        for (int db = 0; db < D / 32; ++db) kf[tt][db] = is_new ? rot[db] : kf[tt][db];
+                        if (rt == 0 && kb + 16 * tt + l == start_pos) {
+                            _Float16* kw = dr.kc + static_cast<size_t>(start_pos) * kv_row + static_cast<size_t>(g) * D + 8 * q;
 #pragma unroll
-                        for (int db = 0; db < D / 32; ++db) *reinterpret_cast<f16x8*>(kw + 32 * db) = rot[db];
+                            for (int db = 0; db < D / 32; ++db) *reinterpret_cast<f16x8*>(kw + 32 * db) = rot[db];
+                        }
+                    }
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        if (rt == 0 && kb + 16 * (j >> 2) + 4 * q + (j & 3) == start_pos) {
+                            _Float16* vw = dr.vc + static_cast<size_t>(start_pos) * kv_row + static_cast<size_t>(g) * D + D / 16 * l;
+                            __builtin_memcpy(__builtin_assume_aligned(vw, D / 8), vd[j], 4 * kVW);
+                        }
+                }
+            }
+            // scores: x[4 tt + v] of key kb + 16 tt + 4 q + v
+            const bool full = kb + kRowsKeys <= vis_all;
+            float x[8];
+            float mx = -INFINITY;
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+                f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int db = 0; db < D / 32; ++db) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[tt][db], qf[db], s, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    float y = s[v] * scale_log2;
+                    if (!full && kb + 16 * tt + 4 * q + v >= row_end) y = -INFINITY;
+                    x[4 * tt + v] = y;
+                    mx = fmaxf(mx, y);
+                }
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            // a row that sees no key of this block keeps its state (its maximum may still be -inf)
+            const bool sees = kb < row_end;
+            const float m_new = sees ? fmaxf(m_run, mx) : m_run;
+            const float corr = sees ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
+            const float base = sees ? m_new - kPScale : 0.0f;
+            float sum = 0.0f;
+            f16x8 ph, pl, pw;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float p = __builtin_amdgcn_exp2f(x[i] - base);
+                sum += p;
+                ph[i] = static_cast<_Float16>(p);
+                pl[i] = static_cast<_Float16>(p - static_cast<float>(ph[i]));
+                if constexpr (kCareful) pw[i] = static_cast<_Float16>(p > 0.0f ? 1.0f : 0.0f);
+            }
+            sum += __shfl_xor(sum, 16, 64);
+            sum += __shfl_xor(sum, 32, 64);
+            l_run = l_run * corr + sum;
+            m_run = m_new;
+#pragma unroll
+            for (int dt = 0; dt < D / 16; ++dt) o[dt] *= corr;
+            // product dt: operand row l is dim D/16 l + dt of the lane's 8 keys
+            if constexpr (!kCareful) {
+#pragma unroll
+                for (int dt = 0; dt < D / 16; ++dt) {
+                    uint32_t t[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        t[i] = __builtin_amdgcn_perm(vd[2 * i + 1][dt >> 1], vd[2 * i][dt >> 1], (dt & 1) ? 0x07060302u : 0x05040100u);
+                    f16x8 vf;
+                    __builtin_memcpy(&vf, t, 16);
+                    o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph, o[dt], 0, 0, 0);
+                    o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl, o[dt], 0, 0, 0);
+                }
+            } else {
+#pragma unroll 1
+                for (int rr = 0; rr < kRowsTile; ++rr) {
+                    const int end = __shfl(row_end, rr, 64);
+#pragma unroll
+                    for (int dt = 0; dt < D / 16; ++dt) {
+                        uint32_t fin[4], inf[4];  // the row's finite values, the others
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            uint32_t u = __builtin_amdgcn_perm(vd[2 * i + 1][dt >> 1], vd[2 * i][dt >> 1], (dt & 1) ? 0x07060302u : 0x05040100u);
+                            const int k = kb + 16 * (i >> 1) + 4 * q + 2 * (i & 1);  // keys k, k + 1
+                            u &= (k < end ? 0xFFFFu : 0u) | (k + 1 < end ? 0xFFFF0000u : 0u);
+                            const uint32_t keep = ((u & 0x7C00u) != 0x7C00u ? 0xFFFFu : 0u) | ((u & 0x7C000000u) != 0x7C000000u ? 0xFFFF0000u : 0u);
+                            fin[i] = u & keep;
+                            inf[i] = u & ~keep;
+                        }
+                        f16x8 vf, vi;
+                        __builtin_memcpy(&vf, fin, 16);
+                        __builtin_memcpy(&vi, inf, 16);
+                        f32x4 t = o[dt];
+                        t = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph, t, 0, 0, 0);
+                        t = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl, t, 0, 0, 0);
+                        t = __builtin_amdgcn_mfma_f32_16x16x32_f16(vi, pw, t, 0, 0, 0);
+                        o[dt] = l == rr ? t : o[dt];
                     }
                 }
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (rt == 0 && kb + 16 * (j >> 2) + 4 * q + (j & 3) == start_pos) {
-                        _Float16* vw = dr.vc + static_cast<size_t>(start_pos) * kv_row + static_cast<size_t>(g) * D + D / 16 * l;
-                        __builtin_memcpy(__builtin_assume_aligned(vw, D / 8), vd[j], 4 * kVW);
-                    }
             }
         }
-        // scores: x[4 tt + v] of key kb + 16 tt + 4 q + v
-        const bool full = kb + kRowsKeys <= vis_all;
-        float x[8];
-        float mx = -INFINITY;
+    };
+    scan(std::false_type{});
+    // An infinite or NaN value makes the plain products NaN where a row does not see it (0 weight) or where
+    // its weight's lo term is 0 or negative: such a wave starts over.
+    bool bad = false;
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int dt = 0; dt < D / 16; ++dt)
 #pragma unroll
-            for (int db = 0; db < D / 32; ++db) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[tt][db], qf[db], s, 0, 0, 0);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                float y = s[v] * scale_log2;
-                if (!full && kb + 16 * tt + 4 * q + v >= row_end) y = -INFINITY;
-                x[4 * tt + v] = y;
-                mx = fmaxf(mx, y);
-            }
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        // a row that sees no key of this block keeps its state (its maximum may still be -inf)
-        const bool sees = kb < row_end;
-        const float m_new = sees ? fmaxf(m_run, mx) : m_run;
-        const float corr = sees ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
-        const float base = sees ? m_new - kPScale : 0.0f;
-        float sum = 0.0f;
-        f16x8 ph, pl;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float p = __builtin_amdgcn_exp2f(x[i] - base);
-            sum += p;
-            ph[i] = static_cast<_Float16>(p);
-            pl[i] = static_cast<_Float16>(p - static_cast<float>(ph[i]));
-        }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
-        l_run = l_run * corr + sum;
-        m_run = m_new;
-#pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) o[dt] *= corr;
-        // product dt: operand row l is dim D/16 l + dt of the lane's 8 keys
-        auto pv = [&](const uint32_t (&v)[8][kVW], f32x4 (&acc)[D / 16]) {
-#pragma unroll
-            for (int dt = 0; dt < D / 16; ++dt) {
-                uint32_t t[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    t[i] = __builtin_amdgcn_perm(v[2 * i + 1][dt >> 1], v[2 * i][dt >> 1], (dt & 1) ? 0x07060302u : 0x05040100u);
-                f16x8 vf;
-                __builtin_memcpy(&vf, t, 16);
-                acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph, acc[dt], 0, 0, 0);
-                acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl, acc[dt], 0, 0, 0);
-            }
-        };
-        bool plain = true;
-        if (!full) {
-            // some row does not see some key: its weight 0 must not meet an infinite or NaN value
-            bool bad = false;
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-#pragma unroll
-                for (int i = 0; i < kVW; ++i)
-                    bad |= (vd[j][i] & 0x7C00u) == 0x7C00u || (vd[j][i] & 0x7C000000u) == 0x7C000000u;
-            plain = __ballot(bad) == 0;
-        }
-        if (plain) {
-            pv(vd, o);
-        } else {
-            // one row at a time, with the values that it does not see cleared
-            for (int rr = 0; rr < kRowsTile; ++rr) {
-                const int end = __shfl(row_end, rr, 64);
-                uint32_t vz[8][kVW];
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-#pragma unroll
-                    for (int i = 0; i < kVW; ++i) vz[j][i] = kb + 16 * (j >> 2) + 4 * q + (j & 3) < end ? vd[j][i] : 0u;
-                f32x4 t[D / 16];
-#pragma unroll
-                for (int dt = 0; dt < D / 16; ++dt) t[dt] = o[dt];
-                pv(vz, t);
-#pragma unroll
-                for (int dt = 0; dt < D / 16; ++dt) o[dt] = l == rr ? t[dt] : o[dt];
-            }
-        }
-    }
+        for (int v = 0; v < 4; ++v) bad |= o[dt][v] != o[dt][v];
+    if (__ballot(bad) != 0) scan(std::true_type{});
 
     // Lane (l, q) holds dims D/4 q + D/16 v + dt of row l in o[dt][v].  Merge of the waves: LDS rows
     // padded by one 16-byte piece.

@@ -79,6 +79,23 @@ def test_rows_ignore_values_they_do_not_see(cuda):
     assert not np.isfinite(got[3:, 4:, 5]).any() and np.isfinite(got[3, :4]).all() and np.isnan(got[4, :4, 9]).all()
 
 
+@pytest.mark.parametrize("q_len,kv_len", [(1, 140), (5, 140), (3, 4000)])
+@pytest.mark.parametrize("d", [64, 128])
+def test_infinite_values_that_a_row_sees(cuda, q_len, kv_len, d):
+    """An infinite value gives an infinite output of its sign, +inf and -inf together NaN, a NaN value NaN, and
+    the other outputs do not change."""
+    Q, K, V = _inputs(q_len, kv_len, 8, 2, d, 5)
+    clean = _run(cuda, Q, K, V, kv_len - q_len, True)
+    V[10, 1, 5] = V[20, 1, 9] = V[100, 1, 50] = np.inf
+    V[40, 1, 7] = V[77, 1, 9] = -np.inf
+    V[33, 1, 11] = np.nan
+    got = _run(cuda, Q, K, V, kv_len - q_len, True)
+    assert (got[:, 4:, [5, 50]] == np.inf).all() and (got[:, 4:, 7] == -np.inf).all() and np.isnan(got[:, 4:, [9, 11]]).all()
+    keep = np.ones(got.shape, bool)
+    keep[:, 4:, [5, 50, 7, 9, 11]] = False
+    assert np.array_equal(got[keep].view(np.uint16), clean[keep].view(np.uint16))
+
+
 @pytest.mark.parametrize("off", [0, 1])
 def test_cache_append_alignment(cuda, off):
     """The new rows reach the cache from 16-byte aligned and from 2-byte aligned sources alike."""
