@@ -886,6 +886,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void attention_rows_kernel(
                     if (k == start_pos) vr = dr.v_new + static_cast<size_t>(g) * D;
                 __builtin_memcpy(vd[j], __builtin_assume_aligned(vr + D / 16 * l, D / 8), 4 * kVW);
             }
+            __builtin_amdgcn_sched_barrier(0);  // every load of the block is out before its first product
             if constexpr (kRope) {
                 if (kb + kRowsKeys > start_pos) {  // the block with the new key
 #pragma unroll
@@ -952,6 +953,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void attention_rows_kernel(
 #pragma unroll
             for (int dt = 0; dt < D / 16; ++dt) o[dt] *= corr;
             // product dt: operand row l is dim D/16 l + dt of the lane's 8 keys
+            __builtin_amdgcn_sched_barrier(0);  // and V's transposition waits for V alone
             if constexpr (!kCareful) {
 #pragma unroll
                 for (int dt = 0; dt < D / 16; ++dt) {
@@ -1001,7 +1003,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void attention_rows_kernel(
     for (int dt = 0; dt < D / 16; ++dt)
 #pragma unroll
         for (int v = 0; v < 4; ++v) bad |= o[dt][v] != o[dt][v];
-    if (__ballot(bad) != 0) scan(std::true_type{});
+    if (__builtin_expect(__ballot(bad) != 0, 0)) scan(std::true_type{});
 
     // Lane (l, q) holds dims D/4 q + D/16 v + dt of row l in o[dt][v].  Merge of the waves: LDS rows
     // padded by one 16-byte piece.
