@@ -1297,8 +1297,9 @@ int attn_chunks(int kv_len) { return kv_len <= 0 ? 1 : (kv_len + kAttnChunk - 1)
 //   kRows: the other calls of head_dim 64 and 128;
 //   kLanes: other head sizes, and Q / K / V that are not 16-byte aligned.
 constexpr int kFaMinRows = 16;
-// Workgroups that a split grid is cut to: two per CU, what the 128-row tile's LDS allows.
-constexpr int64_t kAttnFill = 512;
+// Workgroups that a split grid is cut to: two per CU, what the 128-row tile's LDS allows.  (The 16-row tile of
+// head_dim 128 that rotates its query fits once per CU; its ranges past 256 run in a second round.)
+constexpr int64_t kAttnFill = 512, kAttnCus = 256;
 enum class AttnKind { kMfma, kRows, kLanes };
 struct AttnPlan {
     AttnKind kind;
@@ -1309,9 +1310,19 @@ struct AttnPlan {
 
 // Keys per range: the key blocks of all row tiles spread over kAttnFill workgroups (a block: 64 keys of
 // the 128-row tile, at least two per range, or 32 keys of each wave of the 16-row tile).  A tile's keys
-// are split only while the grid leaves half of the workgroups' places empty: partial results cost
-// 4 D bytes of traffic per row, range and direction.  40 positions of 32 heads over 12040 keys (16
-// row tiles of 128): 27 us and 6.8 us of merge in 32 ranges, against 405 us unsplit.
+// are split only while the grid leaves half of the workgroups' places empty, and where that saves more
+// than it costs:
+//   saved  the longest tile's blocks, 1.6 / 1.0 us each in the 128-row tile (head_dim 128 / 64; 1.4 times
+//          that with two workgroups on a CU) and 1.6 / 0.8 us in the 16-row tile;
+//   cost   the merge, 4.5 us after the 128-row tile (launch gap and more ranges per CU) and 2.5 us after the
+//          16-row tile, and the partial results, written and read at 5 TB/s.
+// us, unsplit / split, 32 heads, 8 of keys, head_dim 128:
+//   200 positions over 200 keys   9.8 / 14.9       400 keys  16.4 / 17.4    3200 keys  ~90 / 30
+//   500 positions over 500 keys  18.1 / 25.0       700 keys  23.1 / 32.7    3500 keys  ~98 / 53.5
+//   1000 positions over 1000 keys 31.8 / 35.6     1200 keys  36.5 / 44.5    4000 keys ~114 / 95
+//   whole 8B decode layer         201 keys 46.5 / 47.5    401 keys 50.0 / 47.3    601 keys 52.6 / 48.6
+// and 4 heads of 64: 40 positions over 240 keys 7.3 / 9.5, 3040 keys 52 / 10; 1B decode layer (32 heads of 64)
+// 201 keys 45.3 / 47.9, 401 keys 47.2 / 47.6, 601 keys 48.3 / 48.1.
 AttnPlan attn_plan(int q_len, int kv_len, int heads, int kv_heads, int head_dim, int start_pos, bool causal, bool aligned,
                    bool may_split) {
     const int group = heads / kv_heads;
@@ -1347,7 +1358,12 @@ AttnPlan attn_plan(int q_len, int kv_len, int heads, int kv_heads, int head_dim,
     if (may_split && 2 * wgs <= kAttnFill) {
         const int64_t even = (blocks * kv_heads + kAttnFill - 1) / kAttnFill;
         const int max_splits = static_cast<int>(2 * kAttnFill / wgs);
-        per = static_cast<int>(std::min<int64_t>(most, std::max<int64_t>({even, mfma ? 2 : 1, (most + max_splits - 1) / max_splits})));
+        const int range = static_cast<int>(std::min<int64_t>(most, std::max<int64_t>({even, mfma ? 2 : 1, (most + max_splits - 1) / max_splits})));
+        const double block_us = head_dim == 128 ? 1.6 : mfma ? 1.0 : 0.8;
+        const double run = static_cast<double>(blocks) / range * kv_heads;  // workgroups that have keys
+        const double part_bytes = static_cast<double>(row_bytes) * blocks / (static_cast<double>(range) * p.tiles);
+        const double saved = block_us * (most - range * (mfma && run > kAttnCus ? 1.4 : 1.0));
+        if (saved > (mfma ? 4.5 : 2.5) + 2.0 * part_bytes / 5e6) per = range;
     }
     p.splits = (most + per - 1) / per;
     p.kps = per * block;

@@ -53,6 +53,16 @@ def test_split_attention(cuda, q_len, kv_len, start, heads, kvh, d, causal):
     assert float(np.abs(got - want).max()) <= bound
 
 
+# both sides of the line between one range and several, last ranges of one key, and ranges that only the
+# last rows of their tile see
+@pytest.mark.parametrize("q_len,kv_len,start,heads,kvh,d,causal", [
+    (1, 640, 639, 32, 8, 128, True), (1, 641, 640, 32, 8, 128, True), (1, 769, 768, 32, 8, 128, True), (1, 1025, 1024, 24, 8, 64, True),
+    (15, 1281, 1266, 64, 8, 128, True), (15, 1281, 1266, 20, 4, 64, True), (16, 257, 241, 8, 8, 128, True), (16, 577, 561, 8, 8, 128, True),
+    (40, 1089, 1049, 32, 8, 64, True), (100, 833, 733, 4, 4, 64, True), (200, 1025, 825, 8, 2, 128, True), (320, 1000, 680, 4, 1, 128, True)])
+def test_split_edges(cuda, q_len, kv_len, start, heads, kvh, d, causal):
+    test_split_attention(cuda, q_len, kv_len, start, heads, kvh, d, causal)
+
+
 @pytest.mark.parametrize("q_len", [3, 40])
 def test_negative_scale(cuda, q_len):
     import torch
