@@ -327,11 +327,13 @@ int qmm_gemm_batch(const qmm_gemm_desc* descs, int count, void* stream) {
             const qmm_gemm_desc& h = descs[i];
             int rc = record(h.ev_before);
             if (rc != QMM_OK) return rc;
-            hipError_t e = h.M >= gmax
-                               ? qmm::launch_gemm_prefill_fused(h.ggml_type, h.A, h.a_dtype, h.c_dtype, h.M, h.K, W, C, N,
-                                                                j - i, s)
-                               : qmm::launch_gemv_fused(h.ggml_type, h.A, h.a_dtype, h.c_dtype, h.M, h.K, W, C, N, j - i, s,
-                                                        ident);
+            // matrices that run different kernels alone do not fuse: the longest run from i that does
+            hipError_t e = hipErrorNotSupported;
+            for (; e == hipErrorNotSupported && j - i >= 2; --j) {
+                e = h.M >= gmax ? qmm::launch_gemm_prefill_fused(h.ggml_type, h.A, h.a_dtype, h.c_dtype, h.M, h.K, W, C, N, j - i, s)
+                                : qmm::launch_gemv_fused(h.ggml_type, h.A, h.a_dtype, h.c_dtype, h.M, h.K, W, C, N, j - i, s, ident);
+                if (e == hipSuccess) break;
+            }
             if (e == hipSuccess) {
                 if ((rc = record(descs[j - 1].ev_after)) != QMM_OK) return rc;
                 i = j;

@@ -1584,10 +1584,11 @@ hipError_t dispatch_types(int t, const void* A, const Seg* segs, int nseg, int M
     // the matrix-core GEMV where it serves the matrix at this M; matrices that run different kernels alone
     // are launched alone
     int kind = 0;
+    const int a_dt = std::is_same<TA, float>::value ? QMM_DTYPE_F32 : QMM_DTYPE_F16;
     if (fast && fz.kind == 0 && fz.ea == nullptr && fz.pair == 0) {
-        kind = gemv_mfma_kind(t, segs[0].W, M, segs[0].N, K, identity);
+        kind = gemv_mfma_kind(t, segs[0].W, M, segs[0].N, K, a_dt, identity);
         for (int j = 1; j < nseg; ++j)
-            if (gemv_mfma_kind(t, segs[j].W, M, segs[j].N, K, identity) != kind) return hipErrorNotSupported;
+            if (gemv_mfma_kind(t, segs[j].W, M, segs[j].N, K, a_dt, identity) != kind) return hipErrorNotSupported;
     }
     if (kind != 0) {
         const void* W[kMaxSegs];
@@ -1598,7 +1599,6 @@ hipError_t dispatch_types(int t, const void* A, const Seg* segs, int nseg, int M
             C[j] = segs[j].C;
             N[j] = segs[j].N;
         }
-        const int a_dt = std::is_same<TA, float>::value ? QMM_DTYPE_F32 : QMM_DTYPE_F16;
         const int c_dt = std::is_same<TC, float>::value ? QMM_DTYPE_F32 : QMM_DTYPE_F16;
         const hipError_t e = launch_gemv_mfma(t, A, a_dt, c_dt, M, K, W, C, N, nseg, kind, stream);
         if (e != hipErrorNotSupported) return e;

@@ -1241,9 +1241,13 @@ hipError_t staged_dispatch(const void* A, const void* const* W, void* const* C, 
     MDev di;
     hipError_t e = mdev(di);
     if (e != hipSuccess) return e;
-    const int passes = (M + kMRows - 1) / kMRows;
+    int passes = (M + kMRows - 1) / kMRows;
     if (passes > 65535) return hipErrorNotSupported;
+    // few row groups: passes of 4 rows and more side by side instead of one wave's loads of 16 (a row's result
+    // does not depend on its pass).  Q4_0 1024 x 4096 at M = 16 11.4 -> 7.6 us, at M = 8 8.8 -> 7.5 us.
+    while (2 * static_cast<int64_t>(nrg) * passes <= di.cus && (M + 2 * passes - 1) / (2 * passes) >= 4) passes *= 2;
     const int lrows = (M + passes - 1) / passes;
+    passes = (M + lrows - 1) / lrows;  // none without rows
     const size_t lds = F::kSlots * (CK::kBytes + kBG * 256 * static_cast<size_t>((lrows + 3) / 4));
     const void* kern = reinterpret_cast<const void*>(&gemv_staged_kernel<F, TA, TC>);
     int occ = 0;
@@ -1278,36 +1282,67 @@ hipError_t mdtypes(int a_dtype, int c_dtype, const void* A, const void* const* W
 
 }  // namespace
 
-// Which kernel serves a matrix.  The choice depends on the matrix and M alone, never on what shares its
-// launch.
+// Which kernel serves a matrix.  The choice depends on the matrix, the activations' type and M alone, never on
+// what shares its launch, so that a batch gives what its matrices give one by one.
 //   Ring kernel.  Q4_K: from M = 2 (v_dot2 is faster at M = 1; 70B gate 28672 x 8192: 26 against 30 us),
 //   and at M = 1 too in row-identity mode.  Q6_K of whole 16-byte rows: from M = 3 (70B down 8192 x 28672:
 //   49-52 us at M = 3, 4 and 55-58 us at M = 8..16 against 41, 42, 72 and 98 us for v_dot2 at M = 1, 2, 4, 8:
 //   its decode takes about 1.5 times the VALU work of Q4_K).
-//   Staged kernel, from 1024 rows on (below, 16-row groups leave most CUs idle and v_dot2's items of one or
-//   two rows are faster at every M).  us against v_dot2, fp16 activations, weights from memory:
-//     Q8_0  4096 x 4096    M = 4: 8.4 / 7.8    M = 8: 9.0 / 11.8   M = 16: 10.3 / 17.2
-//           14336 x 4096   M = 3: 18.8 / 20.1  M = 8: 19.8 / 30.3  M = 16: 22.1 / 45.7
-//     Q4_0  4096 x 4096    M = 4: 8.2 / 6.5    M = 8: 9.4 / 9.8    M = 16: 11.9 / 14.4
-//           14336 x 4096   M = 3: 12.2 / 15.6  M = 8: 13.2 / 25.3  M = 16: 15.8 / 39.9
-//     F16   4096 x 4096    M = 2: 10.3 / 10.6  M = 8: 11.0 / 17.2  M = 16: 11.9 / 27.0
-//           14336 x 4096   M = 3: 23.6 / 35.6  M = 8: 23.8 / 55.9  M = 16: 24.6 / 76.3
-//     Q6_K  4096 x 14080   M = 4: 19.6 / 20.0  M = 8: 19.5 / 30.3  M = 16: 23.8 / 55.3
-//   so F16 from M = 3; the others from M = 5, Q8_0 and Q4_0 from M = 3 where the weights, not the launch, set
-//   the time (2^25 of them; Q4_0 with 8192 rows and more, which fill the CUs).
+//   Staged kernel.  us, v_dot2 / staged, fp16 activations, weights from memory, N x K:
+//                       M = 3         M = 5         M = 8         M = 12        M = 16
+//     Q8_0   512 x 4096 6.2 / 6.4    10.2 / 6.6    10.7 / 6.5     6.4 / 6.9    10.8 / 6.6
+//           1024 x 4096 6.4 / 6.4    10.2 / 6.7    10.7 / 6.7     9.2 / 7.0    10.7 / 6.8
+//           4096 x 4096 7.7 / 8.4    11.3 / 8.7    11.9 / 9.0    17.1 / 9.4    17.5 / 10.2
+//           8192 x 8192  21 / 21      28 / 22       29 / 24       45 / 26       47 / 29
+//          14336 x 4096  20 / 19      28 / 19       30 / 20       40 / 21       45 / 22
+//     Q4_0   512 x 4096 4.4 / 6.9     8.7 / 7.7     9.1 / 7.4     4.7 / 8.3     9.1 / 7.5
+//           1024 x 4096 4.6 / 6.9     8.7 / 7.8     9.2 / 7.5     6.3 / 8.3     9.1 / 7.6
+//           2048 x 4096 4.6 / 7.0     8.7 / 7.9     9.2 / 7.6     8.8 / 8.4     9.2 / 8.8
+//           8192 x 8192  16 / 15      24 / 16       24 / 17       40 / 20       41 / 22
+//          14336 x 4096  16 / 12      25 / 13       26 / 13       36 / 15       40 / 16
+//     F16   1024 x 4096 6.1 / 6.4     6.0 / 6.8     6.2 / 6.7     8.8 / 7.0     9.0 / 6.8
+//           2048 x 4096 7.7 / 8.3    10.0 / 8.6    10.5 / 8.5    13.5 / 8.8    15.5 / 8.9
+//           3072 x 4096  11 / 9.2      15 / 9.6      15 / 9.8      21 / 10       21 / 11
+//     Q6_K   512 x 4352 6.7 / 7.5    13.8 / 7.8    14.2 / 7.8     6.8 / 8.1    14.2 / 7.9
+//           4096 x 14080 20 / 19      30 / 19       30 / 20       52 / 21       56 / 24
+//   (v_dot2 takes 8 rows per block at M = 5..8 and 13..16, where its latency grows most, else 4 or fewer.)
+//   Q8_0, Q4_0, Q6_K: from M = 5; at M = 9..12 and above 16 from 1024 rows on.  At 9..12 v_dot2 is up to
+//   40 % faster on a lone Q4_0 matrix of 1024 rows, but q, k, v of 4096, 1024 and 1024 rows take one launch
+//   of 12 us instead of one of 18 us, and would take two of 19 us if only q came here.
+//   Q8_0 and Q4_0 at M = 3, 4: where the weights set the time (2^25 of them) and the matrix is gate- or
+//   down-shaped; square ones share their activations with k and v, whose own launch costs more than the 1 us saved.
+//   F16: from M = 3, 3072 rows on, or 1024 rows with K > 2048: a lone matrix of 1024 rows is up to 18 % slower and
+//   8B q, k, v take 14 us for 28 at M = 5 (13 for 19 at M = 3); of 2048 x 2048, q, k and v of 512 rows are better off
+//   together on v_dot2 (7.2 us at M = 3 against 11.4 in two launches).
+//   fp32 activations are read twice and scaled by every row group, so v_dot2, which stages them once per
+//   workgroup, stays ahead up to far more rows: Q8_0 4096 x 4096 at M = 5 14.2 / 17.7, 1024 x 14336 18.2 / 50, 28672 x
+//   8192 85 / 80; Q4_0 4096 x 14336 34.5 / 35.2, 6144 x 8192 32 / 23; F16 2048 x 8192 21.3 / 23.6, 4096 x 8192 34 / 31 (M = 3:
+//   22 / 29, 6144 rows 37 / 34); Q6_K 8192 x 14080 at M = 8 65 / 77, 14336 x 14080 108 / 95.
 // Row-identity mode keeps every format but Q4_K on v_dot2 for every M, so that M = 1 calls (decode) keep the
 // faster kernel.
-int gemv_mfma_kind(int ggml_type, const void* W, int M, int N, int K, bool identity) {
+int gemv_mfma_kind(int ggml_type, const void* W, int M, int N, int K, int a_dtype, bool identity) {
     const uintptr_t wa = reinterpret_cast<uintptr_t>(W);
     if (N < 1 || K < 1) return 0;
     // ring kernel: chunks are copied in 16-byte pieces, so rows must be whole pieces
     if (ggml_type == QMM_TYPE_Q4_K) return M >= (identity ? 1 : 2) && wa % 16 == 0 && K % 256 == 0 ? 1 : 0;
     if (identity || M < 3) return 0;
     if (ggml_type == QMM_TYPE_Q6_K && wa % 16 == 0 && K % 2048 == 0) return 1;
-    if (N < 1024 || wa % 2 != 0 || K % (ggml_type == QMM_TYPE_Q6_K ? 256 : 32) != 0) return 0;
-    const bool large = static_cast<int64_t>(N) * K >= int64_t{1} << 25;
-    const bool early = ggml_type == QMM_TYPE_F16 || (large && (ggml_type == QMM_TYPE_Q8_0 || (ggml_type == QMM_TYPE_Q4_0 && N >= 8192)));
-    return M >= (early ? 3 : 5) ? 2 : 0;
+    if (wa % 2 != 0 || K % (ggml_type == QMM_TYPE_Q6_K ? 256 : 32) != 0) return 0;
+    const bool f16w = ggml_type == QMM_TYPE_F16, q4_0 = ggml_type == QMM_TYPE_Q4_0;
+    int min_rows;
+    if (a_dtype == QMM_DTYPE_F32) {
+        if (M < 5) min_rows = f16w ? 6144 : INT_MAX;
+        else min_rows = f16w ? 4096 : q4_0 ? 6144 : ggml_type == QMM_TYPE_Q6_K ? 12288 : 20480;
+    } else if (f16w) {
+        min_rows = K > 2048 ? 1024 : 3072;
+    } else if (M >= 5) {
+        min_rows = (M >= 9 && M <= 12) || M > 16 ? 1024 : 1;
+    } else {
+        const bool large = static_cast<int64_t>(N) * K >= int64_t{1} << 25;
+        if (ggml_type == QMM_TYPE_Q6_K || !large || N == K) return 0;
+        min_rows = N > K ? 10240 : q4_0 ? 8192 : 3072;
+    }
+    return N >= min_rows ? 2 : 0;
 }
 
 hipError_t launch_gemv_mfma(int ggml_type, const void* A, int a_dtype, int c_dtype, int M, int K, const void* const* W,

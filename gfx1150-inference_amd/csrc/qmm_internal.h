@@ -99,10 +99,10 @@ hipError_t launch_gemv_ex(int ggml_type, const void* A, int c_dtype, int M, int 
 int gemv_max_fused();
 // Matrix-core GEMV (qmm_gemv_mfma.hip) for the GEMV family's M, `count` (1..4) matrices sharing the
 // activations.  gemv_mfma_kind: the kernel that serves a matrix at M, 1 the LDS-ring kernel (Q4_K, Q6_K), 2 the
-// register-staged kernel (Q8_0, Q4_0, F16, Q6_K), 0 neither (v_dot2); it depends on the matrix and M alone,
-// and matrices of one launch must agree.  launch_gemv_mfma: `kind` as that returns it; hipErrorNotSupported
-// when the shape is outside the kernel.
-int gemv_mfma_kind(int ggml_type, const void* W, int M, int N, int K, bool identity);
+// register-staged kernel (Q8_0, Q4_0, F16, Q6_K), 0 neither (v_dot2); it depends on the matrix, the activations'
+// type and M alone, and matrices of one launch must agree.  launch_gemv_mfma: `kind` as that returns it;
+// hipErrorNotSupported when the shape is outside the kernel.
+int gemv_mfma_kind(int ggml_type, const void* W, int M, int N, int K, int a_dtype, bool identity);
 hipError_t launch_gemv_mfma(int ggml_type, const void* A, int a_dtype, int c_dtype, int M, int K, const void* const* W,
                             void* const* C, const int* N, int count, int kind, hipStream_t stream);
 hipError_t launch_gemm_prefill(int ggml_type, const void* A, int a_dtype, const void* W, void* C,

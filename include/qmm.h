@@ -66,12 +66,13 @@ size_t qmm_weight_bytes(int ggml_type, int64_t n, int64_t k);
  * M < qmm_gemv_max_m() (17) runs the bandwidth-bound GEMV kernels; larger M runs the f16-MFMA
  * prefill GEMM (a 32-row tile up to M = 32), whose rows agree with the M = 1 call within the
  * prefill accuracy bound.  Among GEMV sizes each matrix takes the faster of two kernel families, by
- * its type, rows and size and by M alone:
+ * its type, alignment, rows and size, the activations' type and M alone:
  *   v_dot2 GEMV       every M below the following;
  *   matrix-core GEMV  Q4_K (16-byte aligned) from M = 2; Q6_K from M = 3 where K is a multiple of 2048 and
- *                     the weights are 16-byte aligned, else from M = 5; F16 from M = 3; Q8_0 and Q4_0 from
- *                     M = 5, or from M = 3 with 2^25 weights and more (Q4_0: and 8192 rows).  All but Q4_K
- *                     and the first Q6_K case: matrices of 1024 rows and more, K a multiple of 32.
+ *                     the weights are 16-byte aligned.  With K a multiple of 32 and fp16 activations: other
+ *                     Q6_K, Q8_0 and Q4_0 from M = 5 (M = 9..12 and above 16: 1024 rows and more), Q8_0 and Q4_0
+ *                     from M = 3 for large matrices that are not square, F16 from M = 3 with 3072 rows and more
+ *                     (1024 where K > 2048).  With fp32 activations: matrices of many thousand rows.
  * Rows are bit-identical for every M within one family, and the two families agree within the GEMV
  * accuracy bound.  With qmm_set_row_identity(1) every GEMV-size M runs one family (Q4_K the
  * matrix-core GEMV, the other formats the v_dot2 GEMV), so that every row is bit-identical to the

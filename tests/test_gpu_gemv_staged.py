@@ -69,3 +69,31 @@ def test_staged_gemv_rows_and_alignment(cuda, t, N, K):
     for M in (5, 6, 9):
         assert np.array_equal(_gemm(cuda, t, raw, x[:M], N, K), full[:M]), M
     assert np.array_equal(_gemm(cuda, t, raw, x, N, K, off=2), full)
+
+
+# Few rows: the activation rows run in passes of four and more beside each other, the last one shorter.
+@pytest.mark.parametrize("t,N,K", [(O.GGML_Q8_0, 16, 2048), (O.GGML_Q8_0, 513, 2080), (O.GGML_Q4_0, 1, 32), (O.GGML_Q4_0, 515, 4640),
+                                   (O.GGML_Q6_K, 33, 2304), (O.GGML_Q6_K, 1000, 256), (F16, 1040, 2080)])
+def test_few_rows_in_several_passes(cuda, t, N, K):
+    raw, x = _case(t, N, K, 16, np.float16, N + K)
+    y64 = _want(t, raw, x, N, K)
+    full = _gemm(cuda, t, raw, x, N, K)
+    assert np.abs(full - y64).max() / np.abs(y64).max() <= 1e-5
+    for M in (5, 7, 8, 13, 14):
+        assert np.array_equal(_gemm(cuda, t, raw, x[:M], N, K), full[:M]), M
+
+
+@pytest.mark.parametrize("M", [17, 20, 33, 40, 100])
+def test_more_rows_than_one_pass(cuda, M):
+    """With the GEMV / prefill threshold raised: passes without a row are not launched."""
+    import qmm
+    t, N, K = O.GGML_Q8_0, 1024, 544
+    raw, x = _case(t, N, K, M, np.float16, M)
+    y64 = _want(t, raw, x, N, K)
+    qmm.set_thread_gemv_max_m(256)
+    try:
+        got = _gemm(cuda, t, raw, x, N, K)
+    finally:
+        qmm.set_thread_gemv_max_m(0)
+    assert np.abs(got - y64).max() / np.abs(y64).max() <= 1e-5
+    assert np.array_equal(got[:16], _gemm(cuda, t, raw, x[:16], N, K))
