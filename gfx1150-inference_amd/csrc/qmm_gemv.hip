@@ -1447,9 +1447,19 @@ hipError_t launch_staged(const void* A, const Seg* segs, int nseg, int M, int K,
         const void* kern = reinterpret_cast<const void*>(&gemv_resident_kernel<F, MR, YT, NW, FU, TA, TC>);
         int occ = 0;
         if ((e = occupancy(kern, threads, res_lds, occ)) != hipSuccess) return e;
-        // Q6_K at M = 1: four waves per SIMD.  Its 80 registers would let six in, which is slower (lm_head
-        // 128256 x 4096: 79 -> 84 us).
-        if constexpr (F::kType == QMM_TYPE_Q6_K && MR == 1) occ = min(occ, max(1, 16 / NW));
+        // At M = 1 four waves per SIMD, though the registers let six or eight in: the grid is sized by them, and
+        // waves that take several rows keep more loads in flight.  us, all that fit / four waves (fp16 activations):
+        //   Q6_K 128256 x 4096 84 / 79;  Q4_0 8192 x 8192 11.0 / 10.2, 14336 x 4096 9.1 / 8.7, 57344 x 8192 52 / 50;
+        //   Q8_0 12288 x 4096 13.6 / 12.4, 14336 x 4096 15.2 / 14.4;  F16 14336 x 2048 15.7 / 14.7, 8192 x 14336 58 / 55.
+        // Exceptions: many Q4_0 rows of half a window (20480 x 2048 10.9 with six, 11.5 with four; 14336 x 2048 8.9 and
+        // 8.4) and the 16-wave workgroups of Q8_0 (14336 x 28672 97.5 with two of them, 99.7 with one).
+        if constexpr (MR == 1 && F::kType == QMM_TYPE_Q6_K) occ = min(occ, max(1, 16 / NW));
+        if constexpr (MR == 1 && !FU && std::is_same<TA, __half>::value) {
+            int rows = 0;
+            for (int j = 0; j < nseg; ++j) rows += segs[j].N;
+            if (F::kType == QMM_TYPE_Q4_0) occ = min(occ, max(1, (K <= kGemvWindow / 2 && rows >= 16384 ? 24 : 16) / NW));
+            if (F::kType == QMM_TYPE_F16 || (F::kType == QMM_TYPE_Q8_0 && NW < 16)) occ = min(occ, max(1, 16 / NW));
+        }
         GemvSegs<TC> sg;
         const int nrg = seg_table<TC, YT>(segs, nseg, fz, sg);
         const int need = (nrg + NW - 1) / NW;
