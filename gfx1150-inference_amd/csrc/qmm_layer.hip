@@ -243,23 +243,23 @@ struct RopeFreq {
 // Rotates pairs of q (n_q heads) into q_out and of k (n_k heads) into k_out, and copies v
 // (n_k heads) into v_out; rows are token positions pos_offset + s.  q_out / k_out / v_out row
 // strides are given in elements (the KV cache rows hold n_k heads).  A thread takes one pair of one
-// position and every `groups`-th head of its block's range, so that an angle's sine and cosine serve all of
-// them (1023 positions of 64 + 8 heads of 128: 15.0 us against 20.8 us with one thread per rotated pair).  Block (s, y):
-// heads [y hpb, y hpb + hpb).
+// position and every hg-th head of its block's range, so that an angle's sine and cosine serve all of
+// them (1023 positions of 64 + 8 heads of 128: 15.0 us against 20.8 us with one thread per rotated pair).
+// Block (x, y): ppb positions from x ppb, more than one where the heads leave threads idle (20000 positions of
+// one head of 128: 7.3 us against 10.6 us with one), heads [y hpb, y hpb + hpb).
 __global__ __launch_bounds__(256) void rope_kernel(const _Float16* q, _Float16* q_out, int n_q, const _Float16* k, _Float16* k_out,
-                                                  const _Float16* v, _Float16* v_out, int n_k, int head_dim, int pos_offset, int neox,
-                                                  int hpb, RopeFreq fr) {
+                                                  const _Float16* v, _Float16* v_out, int n_k, int seq_len, int head_dim, int pos_offset,
+                                                  int neox, int hpb, int hg, int ppb, RopeFreq fr) {
     const int half_dim = head_dim / 2;
-    const int groups = 256 / half_dim;  // heads at a time (half_dim <= 128)
     const int p = threadIdx.x % half_dim, gi = threadIdx.x / half_dim;
-    if (gi >= groups) return;
-    const int s = blockIdx.x;
+    const int s = blockIdx.x * ppb + gi / hg;
+    if (gi >= hg * ppb || s >= seq_len) return;
     const float ang = static_cast<float>(pos_offset + s) * fr.inv[p];
     const float c = cosf(ang), sn = sinf(ang);
     const int i0 = neox ? p : 2 * p;
     const int i1 = neox ? p + half_dim : 2 * p + 1;
     const int end = min(n_q + n_k, static_cast<int>(blockIdx.y + 1) * hpb);
-    for (int hh = blockIdx.y * hpb + gi; hh < end; hh += groups) {
+    for (int hh = blockIdx.y * hpb + gi % hg; hh < end; hh += hg) {
         const _Float16* src;
         _Float16* dst;
         if (hh < n_q) {
@@ -1437,13 +1437,15 @@ hipError_t launch_rope(const void* q, void* q_out, int n_q, const void* k, void*
     for (int i = 0; i < head_dim / 2; ++i)
         fr.inv[i] = 1.0f / std::pow(freq_base, static_cast<float>(2 * i) / static_cast<float>(head_dim));
     // heads per block: as many as leave about 2048 blocks, at least one pass of the block's threads
-    const int heads = n_q + n_k, groups = 256 / (head_dim / 2);
+    const int heads = n_q + n_k, groups = 256 / (head_dim / 2);  // rotated heads that a block holds at a time
+    const int hg = std::min(groups, heads), ppb = groups / hg;
     const int64_t want = (static_cast<int64_t>(heads) * seq_len + 2047) / 2048;
-    const int hpb = static_cast<int>(std::min<int64_t>(heads, std::max<int64_t>(want, groups)));
-    hipLaunchKernelGGL(rope_kernel, dim3(static_cast<unsigned>(seq_len), static_cast<unsigned>((heads + hpb - 1) / hpb)), dim3(256), 0, stream,
+    const int hpb = static_cast<int>(std::min<int64_t>(heads, std::max<int64_t>(want, hg)));
+    hipLaunchKernelGGL(rope_kernel, dim3(static_cast<unsigned>((seq_len + ppb - 1) / ppb), static_cast<unsigned>((heads + hpb - 1) / hpb)),
+                       dim3(256), 0, stream,
                        static_cast<const _Float16*>(q), static_cast<_Float16*>(q_out), n_q, static_cast<const _Float16*>(k),
                        static_cast<_Float16*>(k_out), static_cast<const _Float16*>(v), static_cast<_Float16*>(v_out), n_k,
-                       head_dim, pos_offset, neox ? 1 : 0, hpb, fr);
+                       seq_len, head_dim, pos_offset, neox ? 1 : 0, hpb, hg, ppb, fr);
     return hipGetLastError();
 }
 

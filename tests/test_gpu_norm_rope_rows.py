@@ -49,3 +49,9 @@ def test_rope_head_blocks(cuda, seq, heads, d, neox):
     qmm.check(qmm.lib().qmm_rope(X.data_ptr(), out.data_ptr(), seq, heads, d, 7, 10000.0, int(neox), torch.cuda.current_stream().cuda_stream))
     torch.cuda.synchronize()
     assert np.abs(out.cpu().numpy().astype(np.float32) - L.rope(x, 7, 10000.0, neox).astype(np.float32)).max() < 4e-3
+
+
+@pytest.mark.parametrize("seq,heads,d,neox", [(1, 1, 128, False), (7, 1, 128, True), (1001, 1, 64, False), (13, 2, 2, True), (9, 5, 64, False), (3, 127, 4, True)])
+def test_rope_few_heads(cuda, seq, heads, d, neox):
+    """Blocks of several positions, the last one not full."""
+    test_rope_head_blocks(cuda, seq, heads, d, neox)
