@@ -451,6 +451,12 @@ __device__ __forceinline__ void vm_wait_rt(int n) {
 }
 __device__ __forceinline__ void lds_sync() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ __forceinline__ void lds_reads_done() { __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// Orders one wave's LDS accesses across its lanes: a wave's LDS operations run in program order, so only the
+// compiler has to keep it (no instruction).
+__device__ __forceinline__ void lds_wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 // Weight chunk of a row group: 16 rows x 8 super-blocks (one per slot), copied row by row into an LDS
 // ring slot of 16 x kRP 16-byte pieces (kRP = the chunk row's pieces, plus one unused piece where that
@@ -1008,9 +1014,11 @@ __global__ __launch_bounds__(64 * F::kSlots, 4) void gemv_staged_kernel(const TA
 #pragma unroll 1
             for (int q = 0; q < bs; ++q) {
                 if (p_fix) fix();
-                // the slot is this wave's own, and a wave's LDS operations run in order
+                // the slot is this wave's own: after the last unit's reads by other lanes, before this one's
+                lds_wave_order();
 #pragma unroll
                 for (int i = 0; i < CK::kIt; ++i) *reinterpret_cast<mu4*>(slot + prow[i] * CK::kRS + pby[i]) = st[i];
+                lds_wave_order();
                 const bool row_end = q + 1 == bs, win_end = row_end && j + 1 == nwin;
                 request(win_end ? b0 + bs : row_end ? b0 : b0 + q + 1, win_end ? 0 : row_end ? j + 1 : j);
                 if (kv > 0) {
