@@ -47,16 +47,16 @@ def test_matrices_that_share_activations_agree(t):
 
 def test_large_matrices_at_three_and_four_rows():
     for t in (Q8_0, Q4_0):
-        assert kind(t, 3, 14336, 4096) == kind(t, 4, 28672, 8192) == kind(t, 3, 8192, 28672) == 2
+        assert kind(t, 3, 14336, 4096) == kind(t, 4, 28672, 8192) == kind(t, 3, 8192, 28672) == kind(t, 4, 14336, 14336) == 2
         assert kind(t, 3, 8192, 8192) == kind(t, 4, 4096, 4096) == kind(t, 3, 8192, 4096) == kind(t, 2, 28672, 8192) == 0
     assert kind(Q8_0, 3, 4096, 14336) == 2 and kind(Q4_0, 3, 4096, 14336) == 0
     assert kind(Q6_K, 4, 28672, 14080) == 0
 
 
 def test_f16_rows():
-    for M in (3, 5, 8, 16):
+    for M in (3, 5, 8, 9, 16):
         assert kind(F16, M, 4096, 4096) == kind(F16, M, 1024, 4096) == kind(F16, M, 3072, 2048) == 2
-        assert kind(F16, M, 2048, 2048) == kind(F16, M, 512, 2048) == kind(F16, M, 1023, 4096) == 0
+        assert kind(F16, M, 2048, 2048) == (2 if M > 8 else 0) and kind(F16, M, 512, 2048) == kind(F16, M, 1023, 4096) == 0
     assert kind(F16, 2, 8192, 8192) == 0
 
 
