@@ -1321,8 +1321,8 @@ hipError_t mdtypes(int a_dtype, int c_dtype, const void* A, const void* const* W
 //   10240 rows (14336 x 14336 Q4_0 46 / 32); smaller square ones share their activations with k and v, whose own
 //   launch costs more than the 1 us saved.
 //   F16: from M = 3, 1024 rows on: a lone matrix of 1024 rows is up to 18 % slower and 8B q, k, v take 14 us for 28 at
-//   M = 5 (13 for 19 at M = 3).  At M <= 8 with K <= 2048 from 3072 rows on: of 2048 x 2048, q, k and v of 512 rows are
-//   better off together on v_dot2 (7.2 us at M = 3 against 11.4 in two launches).
+//   M = 5 (13 for 19 at M = 3).  With K <= 2048 from 3072 rows on: of 2048 x 2048, q, k and v of 512 rows are better off
+//   together on v_dot2 (7.2 us at M = 3 and 9.0 at M = 5 against 11.4 and 11.7 in two launches).
 //   fp32 activations are read twice and scaled by every row group, so v_dot2, which stages them once per
 //   workgroup, stays ahead up to far more rows: Q8_0 4096 x 4096 at M = 5 14.2 / 17.7, 1024 x 14336 18.2 / 50, 28672 x
 //   8192 85 / 80; Q4_0 4096 x 14336 34.5 / 35.2, 6144 x 8192 32 / 23; F16 2048 x 8192 21.3 / 23.6, 4096 x 8192 34 / 31 (M = 3:
@@ -1343,7 +1343,7 @@ int gemv_mfma_kind(int ggml_type, const void* W, int M, int N, int K, int a_dtyp
         if (M < 5) min_rows = f16w ? 6144 : INT_MAX;
         else min_rows = f16w ? 4096 : q4_0 ? 6144 : ggml_type == QMM_TYPE_Q6_K ? 12288 : 20480;
     } else if (f16w) {
-        min_rows = K > 2048 || M > 8 ? 1024 : 3072;
+        min_rows = K > 2048 ? 1024 : 3072;
     } else if (M >= 5) {
         min_rows = (M >= 9 && M <= 12) || M > 16 ? 1024 : 1;
     } else {

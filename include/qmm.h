@@ -72,8 +72,7 @@ size_t qmm_weight_bytes(int ggml_type, int64_t n, int64_t k);
  *                     the weights are 16-byte aligned.  With K a multiple of 32 and fp16 activations: other
  *                     Q6_K, Q8_0 and Q4_0 from M = 5 (M = 9..12 and above 16: 1024 rows and more), Q8_0 and Q4_0
  *                     from M = 3 for large matrices with K > N or many rows, F16 from M = 3 with 1024 rows and
- *                     more (3072 where K <= 2048 and M <= 8).  With fp32 activations: matrices of many thousand
- *                     rows.
+ *                     more (3072 where K <= 2048).  With fp32 activations: matrices of many thousand rows.
  * Rows are bit-identical for every M within one family, and the two families agree within the GEMV
  * accuracy bound.  With qmm_set_row_identity(1) every GEMV-size M runs one family (Q4_K the
  * matrix-core GEMV, the other formats the v_dot2 GEMV), so that every row is bit-identical to the

@@ -56,7 +56,7 @@ def test_large_matrices_at_three_and_four_rows():
 def test_f16_rows():
     for M in (3, 5, 8, 9, 16):
         assert kind(F16, M, 4096, 4096) == kind(F16, M, 1024, 4096) == kind(F16, M, 3072, 2048) == 2
-        assert kind(F16, M, 2048, 2048) == (2 if M > 8 else 0) and kind(F16, M, 512, 2048) == kind(F16, M, 1023, 4096) == 0
+        assert kind(F16, M, 2048, 2048) == kind(F16, M, 512, 2048) == kind(F16, M, 1023, 4096) == 0
     assert kind(F16, 2, 8192, 8192) == 0
 
 
