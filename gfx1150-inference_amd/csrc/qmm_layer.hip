@@ -997,12 +997,13 @@ __global__ __launch_bounds__(64 * kRowsWaves) void attention_rows_kernel(
     };
     scan(std::false_type{});
     // An infinite or NaN value makes the plain products NaN where a row does not see it (0 weight) or where
-    // its weight's lo term is 0 or negative: such a wave starts over.
+    // its weight's lo term is 0 or negative: such a wave starts over, unless the scores themselves are NaN.
     bool bad = false;
 #pragma unroll
     for (int dt = 0; dt < D / 16; ++dt)
 #pragma unroll
         for (int v = 0; v < 4; ++v) bad |= o[dt][v] != o[dt][v];
+    bad = bad && l_run == l_run;
     if (__builtin_expect(__ballot(bad) != 0, 0)) scan(std::true_type{});
 
     // Lane (l, q) holds dims D/4 q + D/16 v + dt of row l in o[dt][v].  Merge of the waves: LDS rows

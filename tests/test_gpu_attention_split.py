@@ -106,6 +106,20 @@ def test_infinite_values_that_a_row_sees(cuda, q_len, kv_len, d):
     assert np.array_equal(got[keep].view(np.uint16), clean[keep].view(np.uint16))
 
 
+@pytest.mark.parametrize("q_len,kv_len", [(3, 140), (3, 4000)])
+def test_nan_scores_stay_with_their_row(cuda, q_len, kv_len):
+    """A NaN query makes its own row NaN; a NaN key every row that sees it."""
+    Q, K, V = _inputs(q_len, kv_len, 8, 2, 128, 6)
+    clean = _run(cuda, Q, K, V, kv_len - q_len, True)
+    Q[1, 2, 7] = np.nan
+    K[kv_len - 1, 1, 3] = np.nan  # the last position's key of the second KV head
+    got = _run(cuda, Q, K, V, kv_len - q_len, True)
+    want_nan = np.zeros(got.shape, bool)
+    want_nan[1, 2] = want_nan[q_len - 1, 4:] = True
+    assert np.array_equal(np.isnan(got), want_nan)
+    assert np.array_equal(got[~want_nan].view(np.uint16), clean[~want_nan].view(np.uint16))
+
+
 @pytest.mark.parametrize("off", [0, 1])
 def test_cache_append_alignment(cuda, off):
     """The new rows reach the cache from 16-byte aligned and from 2-byte aligned sources alike."""
