@@ -682,9 +682,10 @@ __device__ __forceinline__ void mac_window(const typename F::Raw (&cur)[YT], int
 // the norm weights, 16-byte vectors), then v is formed, v^2 is reduced over the workgroup for the
 // norm kinds, and the staged fp16 pairs and sums are written as StageItem::store does.
 // A lane's vectors lie 32 or 64 bytes apart, so each load instruction takes the address unit 32 to 64
-// cycles: only the waves that hold items load (K = 4096 has items for 4 of 8 waves), and the loads go out
-// before the first weights, which return behind them.  8B decode q/k/v 13.1 -> 7.4 us, gate/up 21.3 ->
-// 16.5 us against loads by every thread for both of its places, behind the weights.
+// cycles: only the waves that hold items load (K = 4096 has items for 4 of 8 waves).  In the resident kernel the
+// loads go out before the first weights, which return behind them; the streamed kernel requests its ring's first
+// windows before.  8B decode q/k/v 13.1 -> 7.4 us, gate/up 21.3 -> 16.5 us (resident) against loads by every thread
+// for both of its places, behind the weights.
 constexpr int kFuseOwn = 2;
 // The folded staging exists for one fp16 activation row (decode) and where its registers fit
 // beside the kernel's own (1024-thread workgroups have 128 per lane: one row per item there,

@@ -700,8 +700,8 @@ __global__ __launch_bounds__(64 * kSlots) void gemv_mfma_kernel(const TA* __rest
 //     (1024 + u) pairs of u = q + 128, v_pk_add_f16 leaves q exactly, and y += d T in fp32.
 //   * Q4_0: quarter c takes code bytes 4c..4c+3 of the block (k 4c.. and 16 + 4c..); q - 8 is exact.
 //   * F16: the operands as they lie.  Q6_K: below.
-// Bound by the weight stream between a start and an end: 16 waves keep 70 KB of Q8_0 in flight per CU
-// (about 6 TB/s), but first data arrive 4-5 us after the launch and the last wave's unit is worth 2 us.
+// Bound by the weight stream between a start and an end: 16 waves keep 70 KB of Q8_0 in flight per CU,
+// but first data arrive 4-5 us after the launch and the last wave's unit is worth 2 us.
 // 16 waves of one row group per CU (Q4_0, F16) or two row groups of 8 (Q8_0, Q6_K), whichever measured
 // faster: 8B steps at M = 8, 4 Q8_0 layers, 291 us against 318; 14336 x 4096 Q4_0 13.2 against 17.3.
 // ------------------------------------------------------------------------------------------------

@@ -236,6 +236,12 @@ int qmm_rope(const void* x_in, void* x_out, int seq_len, int num_heads, int head
 /* Grouped-query attention: Q [q_len, num_heads, head_dim], K / V [kv_len, num_kv_heads, head_dim],
  * query head h reads KV head h / (num_heads / num_kv_heads); causal rows m see keys
  * < min(kv_len, start_pos + m + 1); scale 0 means 1 / sqrt(head_dim); head_dim <= 256.
+ * A call whose keys are split over workgroups uses a per-(device, stream) scratch that grows with
+ * q_len and kv_len; calls of several host threads on one stream take turns on it.  Under stream
+ * capture, and on hipStreamPerThread, calls of 16 rows and more (head_dim 64 and 128) do not split:
+ * their fp32 sums are then in another order than an eager call's.  Captured calls of fewer rows use
+ * the scratch: run the largest one eagerly on the stream first, and keep qmm_release_workspace()
+ * for after the graph.
  * Replaces launch_gqa_attention_fp16 (src/kernels/attention.hip:228-284). */
 int qmm_gqa_attention(const void* Q, const void* K, const void* V, void* out, int q_len, int kv_len, int num_heads,
                       int num_kv_heads, int head_dim, int start_pos, float scale, int causal, void* stream);
@@ -361,8 +367,9 @@ int qmm_read_file(const char* path, const qmm_file_range* ranges, int count, int
 
 /* Release the host-API workspace (the reference frees its static Q4Workspace at exit,
  * dequantize.hip:715-719) and the prefill workspaces of qmm_gemm (f16 activations, split-K
- * partials; grow-only per device and stream).  Synchronizes each device that holds one, so it
- * is safe to call at any time; the next call that needs a workspace re-grows it. */
+ * partials; grow-only per device and stream) and of the layer and attention calls.  Waits for calls
+ * that are being issued on one of the latter and synchronizes each device that holds a workspace;
+ * the next call that needs one re-grows it. */
 int qmm_release_workspace(void);
 
 #ifdef __cplusplus
