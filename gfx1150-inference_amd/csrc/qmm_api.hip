@@ -6,11 +6,98 @@
 // reference's std::invalid_argument), a HIP failure is QMM_ERR_HIP (std::runtime_error).
 #include <atomic>
 #include <cmath>
+#include <map>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <unordered_map>
+#include <utility>
+#include <vector>
 
 #include "qmm_internal.h"
+
+namespace qmm {
+namespace {
+
+// A call keeps the entry of its workspace locked from the moment it takes the buffer until its last launch that
+// uses it is enqueued: calls of several host threads on one stream then use the buffer one after the other, in
+// stream order, and neither a larger call nor qmm_release_workspace() frees a buffer that a call holds but has
+// not launched with.  Entries are never erased, so a reference stays valid without the map's lock.
+struct DeviceWorkspace {
+    std::mutex mu;
+    void* buf = nullptr;
+    size_t cap = 0;
+    uint64_t owner = 0;  // hipStreamPerThread: the thread that used it last
+};
+std::mutex g_workspaces_mutex;
+std::map<std::tuple<WorkspaceKind, int, uintptr_t>, DeviceWorkspace> g_workspaces;  // by kind, device and stream handle
+
+uint64_t this_thread_number() {
+    static std::atomic<uint64_t> next{1};
+    thread_local const uint64_t mine = next.fetch_add(1);
+    return mine;
+}
+
+// The runtime owns the pointer from here on, whatever the free reports.
+hipError_t free_workspace(DeviceWorkspace& ws) {
+    void* old = ws.buf;
+    ws.buf = nullptr;
+    ws.cap = 0;
+    return hipFree(old);
+}
+
+}  // namespace
+
+hipError_t take_workspace(WorkspaceKind kind, hipStream_t stream, size_t bytes, std::unique_lock<std::mutex>& held, void** out) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    DeviceWorkspace* ws;
+    {
+        std::lock_guard<std::mutex> lock(g_workspaces_mutex);
+        ws = &g_workspaces[{kind, dev, reinterpret_cast<uintptr_t>(stream)}];
+    }
+    held = std::unique_lock<std::mutex>(ws->mu);
+    if (stream == hipStreamPerThread) {
+        // one handle, a stream for every thread: the previous thread's launches end first
+        if (ws->buf && ws->owner != this_thread_number() && (e = hipDeviceSynchronize()) != hipSuccess) return e;
+        ws->owner = this_thread_number();
+    }
+    if (ws->cap < bytes) {
+        // the previous buffer may still be read by queued work on this stream
+        if (ws->buf && ((e = hipStreamSynchronize(stream)) != hipSuccess || (e = free_workspace(*ws)) != hipSuccess)) return e;
+        if ((e = hipMalloc(&ws->buf, bytes)) != hipSuccess) {
+            ws->buf = nullptr;
+            return e;
+        }
+        ws->cap = bytes;
+    }
+    *out = ws->buf;
+    return hipSuccess;
+}
+
+hipError_t release_workspaces() {
+    int cur = 0;
+    hipError_t e = hipGetDevice(&cur);
+    if (e != hipSuccess) return e;
+    std::vector<std::pair<int, DeviceWorkspace*>> all;
+    {
+        std::lock_guard<std::mutex> lock(g_workspaces_mutex);
+        for (auto& kv : g_workspaces) all.emplace_back(std::get<1>(kv.first), &kv.second);
+    }
+    for (auto& [dev, ws] : all) {
+        std::lock_guard<std::mutex> lock(ws->mu);  // no call is between taking the buffer and its launches
+        if (!ws->buf) continue;
+        if ((e = hipSetDevice(dev)) == hipSuccess && (e = hipDeviceSynchronize()) == hipSuccess) e = free_workspace(*ws);
+        if (e != hipSuccess) {
+            (void)hipSetDevice(cur);  // the first error is the one reported
+            return e;
+        }
+    }
+    return hipSetDevice(cur);
+}
+
+}  // namespace qmm
 
 namespace {
 
@@ -443,7 +530,7 @@ int qmm_gqa_attention(const void* Q, const void* K, const void* V, void* out, in
                                                      causal != 0, may_split);
     hipError_t e;
     std::unique_lock<std::mutex> held;  // until the merge is enqueued
-    if (pb > 0 && (e = qmm::attention_scratch(s, pb, held, &part)) != hipSuccess) return hip_fail(e, "attention workspace");
+    if (pb > 0 && (e = qmm::take_workspace(qmm::WorkspaceKind::kAttention, s, pb, held, &part)) != hipSuccess) return hip_fail(e, "attention workspace");
     const float sc = scale != 0.0f ? scale : 1.0f / std::sqrt(static_cast<float>(head_dim));
     e = qmm::launch_attention(Q, K, V, out, part, q_len, kv_len, num_heads, num_kv_heads, head_dim, start_pos, sc,
                               causal != 0, may_split, s);
@@ -575,8 +662,8 @@ int qmm_dequantize_q6_k_host(const void* q, void* out, int n) { return dequant_h
 int qmm_release_workspace(void) {
     qmm::release_upload_staging();
     {
-        hipError_t le = qmm::release_layer_workspaces();
-        if (le != hipSuccess) return hip_fail(le, "releasing the layer workspaces");
+        hipError_t le = qmm::release_workspaces();
+        if (le != hipSuccess) return hip_fail(le, "releasing the workspaces");
         if ((le = qmm::release_host_staging()) != hipSuccess) return hip_fail(le, "releasing the host staging buffer");
     }
     std::lock_guard<std::mutex> lock(g_ws_mutex);
@@ -593,7 +680,6 @@ int qmm_release_workspace(void) {
     }
     g_ws.clear();
     if ((e = hipSetDevice(cur)) != hipSuccess) return hip_fail(e, "hipSetDevice");
-    if ((e = qmm::release_prefill_workspaces()) != hipSuccess) return hip_fail(e, "release prefill workspace");
     return QMM_OK;
 }
 

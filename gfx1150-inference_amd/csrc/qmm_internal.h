@@ -121,9 +121,6 @@ int prefill_max_fused();
 constexpr size_t kNoAllocScratchBytes = size_t{64} << 20;
 hipError_t launch_gemm_prefill_noalloc(int ggml_type, const void* A, int a_dtype, const void* W, void* C, int c_dtype,
                                        int M, int N, int K, hipStream_t stream, size_t* need);
-// Frees the prefill workspaces (f16 activations, split-K partials) of every device, after
-// synchronizing each device.
-hipError_t release_prefill_workspaces();
 hipError_t launch_embed(int ggml_type, const void* table, int64_t n_rows, int64_t row_bytes, int hidden,
                         const int64_t* ids, int64_t n_ids, void* out, int out_dtype, int* bad, hipStream_t stream);
 hipError_t launch_dequantize(int ggml_type, const void* W, void* out, int out_dtype,
@@ -164,9 +161,12 @@ LayerStatus kv_cache_layer(int layer, int start, int q_len, int kv_heads, int he
                            int* max_seq);
 LayerStatus forward_layer(const qmm_layer_config& cfg, const qmm_layer_weights& w, const void* x_in, void* x_out,
                           int layer_idx, int seq_len, int pos_offset, hipStream_t stream);
-// The attention entry points' scratch of `stream`: the caller keeps `held` until its last launch that uses the
-// buffer is enqueued.
-hipError_t attention_scratch(hipStream_t stream, size_t bytes, std::unique_lock<std::mutex>& held, void** out);
-hipError_t release_layer_workspaces();
+// Grow-only device buffers per kind, device and stream (qmm_api.hip): the prefill GEMM's f16 activations and
+// partial tiles, the layer pipeline's activations, and the standalone attention calls' partial results.  The caller
+// keeps `held` until its last launch that uses the buffer is enqueued.
+enum class WorkspaceKind { kPrefill, kLayer, kAttention };
+hipError_t take_workspace(WorkspaceKind kind, hipStream_t stream, size_t bytes, std::unique_lock<std::mutex>& held, void** out);
+// Frees them all, each once no call holds it, after synchronizing its device.
+hipError_t release_workspaces();
 
 }  // namespace qmm

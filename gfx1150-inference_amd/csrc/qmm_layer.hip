@@ -22,13 +22,10 @@
 //     kernels on the caller's stream with no host synchronisation; activations live in a
 //     grow-only per-(device, stream) workspace.
 #include <algorithm>
-#include <atomic>
 #include <cmath>
-#include <map>
 #include <mutex>
 #include <string>
 #include <unordered_map>
-#include <utility>
 #include <vector>
 
 #include "qmm_device.h"
@@ -624,62 +621,6 @@ struct KvPool {
 };
 std::mutex g_kv_mutex;
 std::unordered_map<int, KvPool> g_kv;
-
-// ---- per-(device, stream) workspaces -----------------------------------------------------------
-// One kind holds the layer pipeline's activations, the other the partial results of the standalone
-// attention entry points (so that they never resize the first).  A call keeps the entry locked from the
-// moment it takes the buffer until its last launch that uses it is enqueued: calls of several host threads
-// on one stream then use the buffer one after the other, in stream order, and neither a larger call nor
-// qmm_release_workspace() frees a buffer that a call holds but has not launched with.  Entries are never
-// erased, so a reference stays valid without the map's lock.
-struct Workspace {
-    std::mutex mu;
-    void* buf = nullptr;
-    size_t cap = 0;
-    uint64_t owner = 0;  // hipStreamPerThread: the thread that used it last
-};
-std::mutex g_ws_map_mutex;
-std::map<std::pair<int, uintptr_t>, Workspace> g_layer_ws, g_scratch_ws;  // by device and stream handle
-
-uint64_t this_thread_number() {
-    static std::atomic<uint64_t> next{1};
-    thread_local const uint64_t mine = next.fetch_add(1);
-    return mine;
-}
-
-hipError_t take_workspace(std::map<std::pair<int, uintptr_t>, Workspace>& map, hipStream_t stream, size_t bytes,
-                          std::unique_lock<std::mutex>& held, void** out) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    Workspace* ws;
-    {
-        std::lock_guard<std::mutex> lock(g_ws_map_mutex);
-        ws = &map[{dev, reinterpret_cast<uintptr_t>(stream)}];
-    }
-    held = std::unique_lock<std::mutex>(ws->mu);
-    if (stream == hipStreamPerThread) {
-        // one handle, a stream for every thread: the previous thread's launches end first
-        if (ws->buf && ws->owner != this_thread_number() && (e = hipDeviceSynchronize()) != hipSuccess) return e;
-        ws->owner = this_thread_number();
-    }
-    if (ws->cap < bytes) {
-        if (ws->buf) {
-            if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;
-            void* old = ws->buf;
-            ws->buf = nullptr;  // the runtime owns the pointer, whatever the free reports
-            ws->cap = 0;
-            if ((e = hipFree(old)) != hipSuccess) return e;
-        }
-        if ((e = hipMalloc(&ws->buf, bytes)) != hipSuccess) {
-            ws->buf = nullptr;
-            return e;
-        }
-        ws->cap = bytes;
-    }
-    *out = ws->buf;
-    return hipSuccess;
-}
 
 // ---- keys split over workgroups ----------------------------------------------------------------
 // Both matrix-core kernels below may cut a row's keys into ranges of `kps` keys, one workgroup each.
@@ -1716,7 +1657,7 @@ LayerStatus forward_layer(const qmm_layer_config& cfg, const qmm_layer_weights& 
     const size_t o_down = take(S * hid * 2), o_part = take(attn_plan(seq_len, kv_len, H, KVH, D, pos_offset, true, attn_aligned(kc, vc, nullptr), true).bytes);
     void* ws_buf = nullptr;
     std::unique_lock<std::mutex> ws_held;  // until the layer's last launch
-    hipError_t e = take_workspace(g_layer_ws, stream, off, ws_held, &ws_buf);
+    hipError_t e = take_workspace(WorkspaceKind::kLayer, stream, off, ws_held, &ws_buf);
     if (e != hipSuccess) return {QMM_ERR_HIP, std::string("layer workspace: ") + hipGetErrorString(e)};
     char* const ws = static_cast<char*>(ws_buf);
     auto fail = [](hipError_t err, const char* what) {
@@ -1875,39 +1816,6 @@ LayerStatus forward_layer(const qmm_layer_config& cfg, const qmm_layer_weights& 
             return fail(e, "residual_add");
     }
     return {QMM_OK, ""};
-}
-
-hipError_t attention_scratch(hipStream_t stream, size_t bytes, std::unique_lock<std::mutex>& held, void** out) {
-    return take_workspace(g_scratch_ws, stream, bytes, held, out);
-}
-
-hipError_t release_layer_workspaces() {
-    int cur = 0;
-    hipError_t e = hipGetDevice(&cur);
-    if (e != hipSuccess) return e;
-    std::vector<std::pair<int, Workspace*>> all;
-    {
-        std::lock_guard<std::mutex> lock(g_ws_map_mutex);
-        for (auto* m : {&g_layer_ws, &g_scratch_ws})
-            for (auto& kv : *m) all.emplace_back(kv.first.first, &kv.second);
-    }
-    for (auto& [dev, ws] : all) {
-        std::lock_guard<std::mutex> lock(ws->mu);  // no call is between taking the buffer and its launches
-        if (!ws->buf) continue;
-        if ((e = hipSetDevice(dev)) != hipSuccess) return e;
-        if ((e = hipDeviceSynchronize()) != hipSuccess) {
-            (void)hipSetDevice(cur);
-            return e;
-        }
-        void* old = ws->buf;
-        ws->buf = nullptr;  // the runtime owns the pointer, whatever the free reports
-        ws->cap = 0;
-        if ((e = hipFree(old)) != hipSuccess) {
-            (void)hipSetDevice(cur);  // the free's error is the one reported
-            return e;
-        }
-    }
-    return hipSetDevice(cur);
 }
 
 }  // namespace qmm

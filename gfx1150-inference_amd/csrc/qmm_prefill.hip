@@ -1438,60 +1438,6 @@ __global__ __launch_bounds__(256) void reduce_kernel(const float* __restrict__ p
     }
 }
 
-// Grow-only device workspace per (device, stream): the f16 copy of the activations and the
-// split-K partial tiles.  Calls on one stream are ordered, so they may share it.
-struct Workspace {
-    void* buf = nullptr;
-    size_t cap = 0;
-};
-std::mutex g_ws_mutex;
-std::unordered_map<std::string, Workspace> g_ws;
-
-hipError_t workspace(hipStream_t stream, size_t bytes, void** out) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    const std::string key = std::to_string(dev) + ":" + std::to_string(reinterpret_cast<uintptr_t>(stream));
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
-    Workspace& ws = g_ws[key];
-    if (ws.cap < bytes) {
-        if (ws.buf) {
-            // the previous buffer may still be read by queued work on this stream
-            if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;
-            if ((e = hipFree(ws.buf)) != hipSuccess) return e;
-            ws.buf = nullptr;
-            ws.cap = 0;
-        }
-        if ((e = hipMalloc(&ws.buf, bytes)) != hipSuccess) return e;
-        ws.cap = bytes;
-    }
-    *out = ws.buf;
-    return hipSuccess;
-}
-
-}  // namespace
-
-hipError_t release_prefill_workspaces() {
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
-    int cur = 0;
-    hipError_t e = hipGetDevice(&cur);
-    if (e != hipSuccess) return e;
-    for (auto& kv : g_ws) {
-        if (!kv.second.buf) continue;
-        const int dev = std::stoi(kv.first.substr(0, kv.first.find(':')));
-        // queued kernels on any stream of the device may still read the buffer
-        if ((e = hipSetDevice(dev)) != hipSuccess) return e;
-        if ((e = hipDeviceSynchronize()) != hipSuccess) return e;
-        if ((e = hipFree(kv.second.buf)) != hipSuccess) return e;
-        kv.second.buf = nullptr;
-        kv.second.cap = 0;
-    }
-    g_ws.clear();
-    return hipSetDevice(cur);
-}
-
-namespace {
-
 int g_cus = 0;
 
 hipError_t cu_count(int& cus) {
@@ -1671,12 +1617,14 @@ hipError_t launch_p(const void* A, const PfSeg* segs, int nseg, int M, int K, hi
     if (plan.ksplit > 1) p_bytes = static_cast<size_t>(plan.ksplit) * M * n_total * 4;
     if (plan.tail_n > 0) p_bytes = static_cast<size_t>(plan.tail_ks) * M * n_tail_total * 4;
     void* ws = nullptr;
+    std::unique_lock<std::mutex> held;  // to the last launch
     if (ext != nullptr) {
         // caller-provided scratch: checked before anything is launched
         ext->need = a_bytes + p_bytes > 0 ? a_bytes + p_bytes + 256 : 0;
         if (ext->need > ext->cap) return hipErrorOutOfMemory;
         ws = ext->buf;
-    } else if (a_bytes + p_bytes > 0 && (e = workspace(stream, a_bytes + p_bytes + 256, &ws)) != hipSuccess) {
+    } else if (a_bytes + p_bytes > 0 &&
+               (e = take_workspace(WorkspaceKind::kPrefill, stream, a_bytes + p_bytes + 256, held, &ws)) != hipSuccess) {
         return e;
     }
     const _Float16* a16 = static_cast<const _Float16*>(A);

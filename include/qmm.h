@@ -368,8 +368,8 @@ int qmm_read_file(const char* path, const qmm_file_range* ranges, int count, int
 /* Release the host-API workspace (the reference frees its static Q4Workspace at exit,
  * dequantize.hip:715-719) and the prefill workspaces of qmm_gemm (f16 activations, split-K
  * partials; grow-only per device and stream) and of the layer and attention calls.  Waits for calls
- * that are being issued on one of the latter and synchronizes each device that holds a workspace;
- * the next call that needs one re-grows it. */
+ * of other threads that are being issued with one, and synchronizes each device that holds one, so it
+ * is safe to call at any time; the next call that needs a workspace re-grows it. */
 int qmm_release_workspace(void);
 
 #ifdef __cplusplus
